@@ -1,0 +1,458 @@
+/*
+ * qmm_gemm.hip -- the stock path for many rows: y[M,N] = x[M,K] . dequant(W)[N,K]^T on the
+ * matrix cores, for one 16-bit dtype of x, scales, biases and y (gfx950).
+ *
+ * The codes enter the MFMAs as exact small integers and everything else stays in fp32, as in
+ * the GEMV: per quantisation group P = sum x (MAGIC + q), y += s * P + b * X - MAGIC * s * X
+ * with X = sum x.  bf16 4-bit codes carry MAGIC = 128 (7 VALU operations make the 8 operands
+ * of a word); fp16 codes take one packed subtraction more and carry none; 8-bit bf16 codes
+ * are converted.
+ *
+ *  - s * P is one fp32 FMA an accumulator element and group: 64 issue cycles a 32 x 32 tile
+ *    against 128 matrix cycles at group 64, so the vector and the matrix pipes run side by
+ *    side.  A group of 128 is taken as two of 64 (the partial sums of a whole tile row would
+ *    not fit in registers).
+ *  - the X terms are a product over groups, so they go through the matrix cores too: X is
+ *    split exactly into three bf16 values (24 bits), and 4 groups x (Xh, Xm, Xl, 0) are the
+ *    16 k slots of one MFMA against b, and of a second against -MAGIC s (or, for fp16, the
+ *    low part of b, split exactly into two bf16 values): one or two MFMAs per 16.
+ *
+ * A workgroup computes 32 RT MW rows x 32 CT NW columns in KW slices of K; a wave holds RT x CT
+ * tiles of one slice.  x is staged in LDS 64 k a step, in two buffers, permuted into the order
+ * of the nibbles and XOR-swizzled by row so that neither writes nor reads conflict; codes are
+ * staged by whole 128-byte lines of their rows (4 or 2 steps), with the line's scales and
+ * biases.  Read straight into the operand registers instead, 32 bytes a row and step, the lines
+ * of 128 columns and their scales outlived the 32 KB L1 and each was fetched several times:
+ * 2048 x 17408, K 5120 took 556 us against 535, 16 x 5120 25.7 against 20.9.  All loads run PD
+ * steps (x) or a line (codes) ahead, and are clamped rather than predicated: with a branch
+ * around them the compiler waited for each at once (636 against 556 us).  KW > 1 slices are
+ * summed through LDS at the end, in slice order.
+ *
+ * Measured on MI355X against the GEMV's launches it replaces (us): 512 x 5120, K 5120, 4-bit
+ * bf16 1537 -> 69; 2048 x 17408, K 5120 12548 -> 535 (682 TFLOP/s); an MLP of 333 rows, 8-bit
+ * fp16 6565 -> 444.  Bound by the chain of a step (staging, LDS reads, MFMAs, FMAs), which two
+ * workgroups a CU overlap only in part: a wave's 64-k step of 128 x 32 needs 576 matrix cycles
+ * and takes about 1600.
+ */
+#include "qmm_device.h"
+#include "qmm_params.h"
+
+namespace {
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+template <bool F16>
+__device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                      __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                       __builtin_bit_cast(bf16x8_t, b), c, 0, 0,
+                                                       0);
+}
+
+/* (1024 + q) pairs -> q pairs, exact. */
+__device__ __forceinline__ uint32_t less_1024(uint32_t v) {
+    const f16x2_t m = {(_Float16)1024.0f, (_Float16)1024.0f};
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2_t, v) - m);
+}
+
+/* fp32 -> the output's dtype, to nearest even (one instruction in either dtype). */
+template <bool F16>
+__device__ __forceinline__ uint16_t round_out(float f) {
+    if constexpr (F16) return __builtin_bit_cast(uint16_t, (_Float16)f);
+    else return __builtin_bit_cast(uint16_t, (__bf16)f);
+}
+
+/* The operand of one word of 4-bit codes, or of two words of 8-bit codes. */
+template <int BITS, bool F16>
+__device__ __forceinline__ u32x4_t code_operand(const uint32_t* w, uint32_t mask,
+                                                uint32_t magic) {
+    u32x4_t v;
+    if constexpr (BITS == 4) {
+        v = nibble_operand<F16>(w[0], mask, magic);
+    } else if constexpr (F16) {
+        v[0] = __builtin_amdgcn_perm(0x64646464u, w[0], 0x04010400u);
+        v[1] = __builtin_amdgcn_perm(0x64646464u, w[0], 0x04030402u);
+        v[2] = __builtin_amdgcn_perm(0x64646464u, w[1], 0x04010400u);
+        v[3] = __builtin_amdgcn_perm(0x64646464u, w[1], 0x04030402u);
+    } else {
+        return byte_operand<false>(w[0], w[1]);
+    }
+    if constexpr (F16)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = less_1024(v[e]);
+    return v;
+}
+
+template <int BITS, int GS, bool F16, int RT, int CT, int MW, int NW, int KW, int PD>
+__device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
+    static_assert(GS == 32 || GS == 64, "sub-groups of a step");
+    constexpr int BM = 32 * RT * MW, BN = 32 * CT * NW;
+    constexpr int NP = 64 / GS;         // groups a step of 64 k holds
+    constexpr int JP = 4 / NP;          // MFMAs a group
+    constexpr int SS = 4 / NP;          // steps of the four groups of an X product
+    constexpr int NWD = BITS;           // code words a lane takes per column and step
+    constexpr int LS = 16 / BITS;       // steps of a 128-byte line of codes
+    constexpr int LG = LS * NP;         // groups of a line
+    constexpr int ST = 64 * MW * NW;    // threads of a slice
+    constexpr int XI = BM * 8 / ST;     // 16-byte chunks of x each of them stages a step
+    constexpr int WI = BN * 8 / ST;     // 16-byte chunks of codes, a line
+    constexpr int SI = 2 * BN > ST ? 2 * BN / ST : 1;  // columns' scales or biases, a line
+    constexpr bool kTwo = F16 || BITS == 4;  // a second X product
+    static_assert(XI * ST == BM * 8 && WI * ST == BN * 8, "whole chunks");
+    static_assert(SI * ST == 2 * BN || SI == 1, "whole rows of scales");
+    static_assert(LS % PD == 0, "a register set per step of a line");
+    /* bytes of a step's x, of four groups' X, of a line of codes and of its scales + biases */
+    constexpr int kA = BM * 128, kX = BM * 32, kW = BN * 128, kS = BN * LG * 4;
+    constexpr int SR = LG == 2 ? 4 : 2;  // lines of scales kept: an X product may need two
+    constexpr int kSlice = 2 * (kA + kX + kW) + SR * kS;
+    constexpr int kRed = (KW - 1) * MW * NW * RT * CT * 4096;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[KW * kSlice > kRed ? KW * kSlice : kRed];
+
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kw = wave / (MW * NW), wn = wave % NW, wm = wave / NW % MW, tl = tid - kw * ST;
+    const int M = p.M, N = p.N, K = p.K, gpr = p.gpr;
+    /* XCD x takes one contiguous run of tiles (rows fastest), so that the row tiles of a
+     * column strip share its codes in one L2 */
+    const int G = gridDim.x;
+    int id = blockIdx.x;
+    if (p.xcd8) {
+        const int x = id & 7, base = G >> 3, rem = G & 7;
+        id = x * base + min(x, rem) + (id >> 3);
+    }
+    const int nt = id / p.tiles_m, m0 = (id - nt * p.tiles_m) * BM, n0 = nt * BN;
+
+    /* the slice's steps, from a fourth one: every slice walks `per` (the barriers are
+     * shared), the last ones may own fewer; loads past K read its last step or line again
+     * and are not used */
+    const int steps = (K + 63) >> 6;
+    const int per = ((steps + KW - 1) / KW + 3) & ~3;
+    const int first = kw * per, mine = min(per, steps - first);
+    const int walk = KW == 1 ? steps : per;
+    uint8_t* abuf = lds + kw * kSlice;
+    uint8_t* xbuf = abuf + 2 * kA;
+    uint8_t* wbuf = xbuf + 2 * kX;
+    uint8_t* sbuf = wbuf + 2 * kW;
+    for (int i = tl; i < 2 * kX / 4; i += ST) ((uint32_t*)xbuf)[i] = 0;  // unused slots
+    const int c8 = tl & 7;
+
+    /* x: chunk c of row r of the tile, rows past M read the last one */
+    const uint8_t* xg = (const uint8_t*)p.x + (size_t)m0 * K * 2;
+    uint32_t xoff[XI];
+    int xr[XI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        xr[i] = (tl + i * ST) >> 3;
+        xoff[i] = (uint32_t)min(xr[i], M - 1 - m0) * (uint32_t)K * 2u + (uint32_t)c8 * 16u;
+    }
+    u32x4_t xv[PD][XI];
+    auto load_x = [&](u32x4_t (&v)[XI], int st) {
+        const uint32_t k0 = (uint32_t)min(first + st, steps - 1) * 64u;
+        const uint8_t* src = xg + (size_t)k0 * 2;
+        /* the half step a K of odd 32s ends in: chunks past it read the half before */
+        const uint32_t back = (GS == 32 && k0 + (uint32_t)c8 * 8u >= (uint32_t)K) ? 64u : 0u;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) v[i] = *(const u32x4_t*)(src + (xoff[i] - back));
+    };
+    auto stage_x = [&](u32x4_t (&v)[XI], int st) {
+        const bool in = GS == 64 || (first + st) * 64 + c8 * 8 < K;
+        uint8_t* ab = abuf + (st & 1) * kA;
+        uint8_t* xb = xbuf + ((st / SS) & 1) * kX;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            if constexpr (GS == 32)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[i][e] = in ? v[i][e] : 0u;
+            *(u32x4_t*)(ab + xr[i] * 128 + ((c8 ^ (xr[i] & 7)) * 16)) =
+                BITS == 4 ? nibble_permute(v[i]) : v[i];
+            float X = chunk_dot<F16>(v[i], 0.0f);
+            X += dpp_f32<0xB1>(X);                             // lanes ^1
+            X += dpp_f32<0x4E>(X);                             // lanes ^2
+            if constexpr (GS == 64) X += dpp_f32<0x141>(X);    // the other half of eight
+            const uint32_t hi = __float_as_uint(X) & 0xffff0000u;
+            const float r1 = X - __uint_as_float(hi);
+            const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
+            const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
+            const int g = (NP == 1) ? (st & 3) : ((st & 1) * 2 + (c8 >> 2));
+            if ((c8 & (GS / 8 - 1)) == 0)
+                *(u32x2_t*)(xb + xr[i] * 32 + g * 8) = u32x2_t{mid | (hi >> 16), lo >> 16};
+        }
+    };
+
+    /* a line of codes: chunk c of column r (the last one past N); chunks past K repeat its
+     * last one */
+    const uint32_t RB = (uint32_t)K * BITS / 8u;
+    const uint8_t* wg = (const uint8_t*)p.w + (size_t)n0 * RB;
+    uint32_t wrow[WI];
+#pragma unroll
+    for (int i = 0; i < WI; ++i) wrow[i] = (uint32_t)min((tl + i * ST) >> 3, N - 1 - n0) * RB;
+    u32x4_t wv[WI];
+    /* scales (items below BN) and biases of a line's groups */
+    uint32_t srow[SI];
+#pragma unroll
+    for (int i = 0; i < SI; ++i)
+        srow[i] = (uint32_t)min((tl + i * ST) % BN, N - 1 - n0) * (uint32_t)gpr;
+    const uint16_t* sg[SI];
+#pragma unroll
+    for (int i = 0; i < SI; ++i)
+        sg[i] = (const uint16_t*)(tl + i * ST < BN ? p.scales : p.biases) + (size_t)n0 * gpr;
+    uint32_t sv[SI][(LG + 1) / 2];
+    auto load_w = [&](int line) {
+        const uint32_t off = min((uint32_t)line * 128u + (uint32_t)c8 * 16u, RB - 16u);
+#pragma unroll
+        for (int i = 0; i < WI; ++i) wv[i] = *(const u32x4_t*)(wg + (wrow[i] + off));
+        if (p.svec) {  // whole lines' groups, aligned: one load
+            const uint32_t g = min((uint32_t)line * LG, (uint32_t)(gpr - LG));
+#pragma unroll
+            for (int i = 0; i < SI; ++i) {
+                const uint16_t* src = sg[i] + (srow[i] + g);
+                if constexpr (LG == 8) {
+                    const u32x4_t v = *(const u32x4_t*)src;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sv[i][e] = v[e];
+                } else if constexpr (LG == 4) {
+                    const u32x2_t v = *(const u32x2_t*)src;
+                    sv[i][0] = v[0];
+                    sv[i][1] = v[1];
+                } else {
+                    sv[i][0] = *(const uint32_t*)src;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < SI; ++i)
+#pragma unroll
+                for (int e = 0; e < LG; e += 2) {
+                    const uint32_t g = (uint32_t)(line * LG + e) >> p.gshift;
+                    const uint32_t g1 = (uint32_t)(line * LG + e + 1) >> p.gshift;
+                    const uint32_t a = sg[i][srow[i] + min(g, (uint32_t)(gpr - 1))];
+                    const uint32_t b = sg[i][srow[i] + min(g1, (uint32_t)(gpr - 1))];
+                    sv[i][e / 2] = a | (b << 16);
+                }
+        }
+    };
+    auto stage_w = [&](int line) {
+        uint8_t* wb = wbuf + (line & 1) * kW;
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int r = (tl + i * ST) >> 3;
+            *(u32x4_t*)(wb + r * 128 + ((c8 ^ (r & 7)) * 16)) = wv[i];
+        }
+        uint32_t* sb = (uint32_t*)(sbuf + (line & (SR - 1)) * kS);
+#pragma unroll
+        for (int i = 0; i < SI; ++i)
+#pragma unroll
+            for (int e = 0; e < LG / 2; ++e)
+                if (SI * ST == 2 * BN || tl < 2 * BN) sb[(tl + i * ST) * (LG / 2) + e] = sv[i][e];
+    };
+
+    f32x16_t acc[RT][CT];
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[r][t][e] = 0.0f;
+    uint32_t magic = F16 ? 0x64006400u : 0x43004300u;
+    uint32_t nmask = 0x000F000Fu;
+    __asm__ volatile("" : "+v"(magic));  // opaque: keep in a VGPR (see nibble_operand)
+    __asm__ volatile("" : "+s"(nmask));  // opaque: keep in an SGPR
+
+    const int line0 = first / LS;
+    /* the X products of the (up to) four groups that end with step st's */
+    auto x_products = [&](int st) {
+        const uint8_t* xb = xbuf + ((st / SS) & 1) * kX;
+        u32x4_t b1[CT], b2[CT];
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+            const int col = (wn * CT + t) * 32 + l32;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                /* the lane half's groups 2h and 2h + 1 of the four; none past K */
+                const int g = st / SS * 4 + 2 * h + e;
+                const uint16_t* sl =
+                    (const uint16_t*)(sbuf + ((line0 + g / LG) & (SR - 1)) * kS) + col * LG +
+                    g % LG;
+                const bool in = (first * NP + g) * GS < K;
+                const uint32_t cs = in ? sl[0] : 0u, cb = in ? sl[BN * LG] : 0u;
+                uint32_t v1, v2;  // the bf16 factors, in the low half
+                if constexpr (F16) {
+                    const float b = elem_to_f32<true>(cb);
+                    const uint32_t bh = __float_as_uint(b) & 0xffff0000u;
+                    v1 = bh >> 16;
+                    v2 = __float_as_uint(b - __uint_as_float(bh)) >> 16;
+                } else {
+                    v1 = cb;
+                    v2 = __float_as_uint(-128.0f * elem_to_f32<false>(cs)) >> 16;
+                }
+                b1[t][2 * e] = v1 | (v1 << 16);
+                b1[t][2 * e + 1] = v1;
+                b2[t][2 * e] = v2 | (v2 << 16);
+                b2[t][2 * e + 1] = v2;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const u32x4_t X =
+                *(const u32x4_t*)(xb + ((wm * RT + r) * 32 + l32) * 32 + h * 16);
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                acc[r][t] = mfma32<false>(X, b1[t], acc[r][t]);
+                if constexpr (kTwo) acc[r][t] = mfma32<false>(X, b2[t], acc[r][t]);
+            }
+        }
+    };
+
+    load_x(xv[0], 0);
+    load_w(line0);
+    __syncthreads();  // the zeroed X slots
+    stage_x(xv[0], 0);
+    stage_w(line0);
+#pragma unroll
+    for (int u = 1; u <= PD; ++u) load_x(xv[u % PD], u);
+
+    for (int l = 0; l * LS < walk; ++l) {
+        const int line = line0 + l;
+#pragma unroll
+        for (int ls = 0; ls < LS; ++ls) {
+            const int st = l * LS + ls;
+            if (st >= walk) break;
+            __syncthreads();  // step st is staged, step st - 1 has been read
+            /* (past the end these read clamped addresses and stage what nothing reads) */
+            stage_x(xv[(ls + 1) % PD], st + 1);
+            load_x(xv[(ls + 1) % PD], st + 1 + PD);
+            if (ls == LS - 1) stage_w(line + 1);
+            if (ls == 0) load_w(line + 1);
+            if (KW > 1 && st >= mine) continue;
+            const uint8_t* wb = wbuf + (line & 1) * kW;
+            const uint16_t* sb = (const uint16_t*)(sbuf + (line & (SR - 1)) * kS);
+            u32x4_t B[CT][4];
+            float s[CT][NP];
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                const int col = (wn * CT + t) * 32 + l32;
+                const uint8_t* row = wb + col * 128;
+                uint32_t w[NWD];
+                constexpr int W = NWD / NP;  // words of a group
+#pragma unroll
+                for (int q = 0; q < NP; ++q) {
+                    /* the lane's words of group q: byte ls * 8 BITS + q * 8 W + h * 4 W */
+                    if constexpr (W == 2) {
+                        const u32x2_t v = *(const u32x2_t*)(
+                            row + (((ls * 2 + q) ^ (col & 7)) * 16 + h * 8));
+                        w[q * W] = v[0];
+                        w[q * W + 1] = v[1];
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < W / 4; ++j) {
+                            const int c = ls * (BITS / 2) + q * (W / 2) + h * (W / 4) + j;
+                            const u32x4_t v = *(const u32x4_t*)(row + ((c ^ (col & 7)) * 16));
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) w[q * W + j * 4 + e] = v[e];
+                        }
+                    }
+                    s[t][q] = elem_to_f32<F16>(sb[col * LG + ls * NP + q]);
+                    if (GS == 32 && (first + st) * 64 + q * GS >= K) s[t][q] = 0.0f;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    B[t][j] = code_operand<BITS, F16>(w + j * NWD / 4, nmask, magic);
+            }
+            const uint8_t* ab = abuf + (st & 1) * kA;
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const uint8_t* row = ab + ((wm * RT + r) * 32 + l32) * 128;
+                u32x4_t A[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int c = (8 / NP) * (j / JP) + JP * h + j % JP;
+                    A[j] = *(const u32x4_t*)(row + ((c ^ (l32 & 7)) * 16));
+                }
+#pragma unroll
+                for (int t = 0; t < CT; ++t)
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) {
+                        f32x16_t P = {};
+#pragma unroll
+                        for (int j = 0; j < JP; ++j)
+                            P = mfma32<F16>(A[q * JP + j], B[t][q * JP + j], P);
+#pragma unroll
+                        for (int e = 0; e < 16; ++e)
+                            acc[r][t][e] = __builtin_fmaf(s[t][q], P[e], acc[r][t][e]);
+                    }
+            }
+            if ((st & (SS - 1)) == SS - 1 || st + 1 == mine) x_products(st);
+        }
+    }
+
+    if constexpr (KW > 1) {  // the other slices' sums to slice 0
+        __syncthreads();
+        f32x4_t* red = (f32x4_t*)lds;
+        constexpr int kV = RT * CT * 4;  // 16-byte values of a lane
+        if (kw > 0) {
+            f32x4_t* o = red + (size_t)((kw - 1) * MW * NW + wm * NW + wn) * kV * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < kV; ++i) {
+                const f32x16_t& a = acc[i / 4 / CT][i / 4 % CT];
+                o[i * 64] = f32x4_t{a[i % 4 * 4], a[i % 4 * 4 + 1], a[i % 4 * 4 + 2],
+                                    a[i % 4 * 4 + 3]};
+            }
+        }
+        __syncthreads();
+        if (kw > 0) return;
+#pragma unroll
+        for (int k2 = 0; k2 < KW - 1; ++k2) {
+            const f32x4_t* o = red + (size_t)(k2 * MW * NW + wm * NW + wn) * kV * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < kV; ++i) {
+                const f32x4_t v = o[i * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[i / 4 / CT][i / 4 % CT][i % 4 * 4 + e] += v[e];
+            }
+        }
+    }
+
+    const uint16_t* lb = (const uint16_t*)p.lbias;
+    uint16_t* y = (uint16_t*)p.y;
+#pragma unroll
+    for (int t = 0; t < CT; ++t) {
+        const int n = n0 + (wn * CT + t) * 32 + l32;
+        if (n >= N) continue;
+        const float add = lb ? elem_to_f32<F16>(lb[n]) : 0.0f;
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + (wm * RT + r) * 32 + (e & 3) + 8 * (e >> 2) + 4 * h;
+                if (m < M) y[(size_t)m * N + n] = round_out<F16>(acc[r][t][e] + add);
+            }
+    }
+}
+
+}  // namespace
+
+#define DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, TILE, RT, CT, MW, NW, KW, PD)                 \
+    extern "C" __global__ void __launch_bounds__(64 * MW * NW * KW, 2)                            \
+        dfq_gemm_b##BITS##_g##GS##_##NAME##_##TILE(QmmGemmParams p) {                        \
+        qmm_gemm<BITS, GS, F16, RT, CT, MW, NW, KW, PD>(p);                                      \
+    }
+/* rows x columns of a workgroup's tile, and slices of K (kGemmTiles in qmm_runtime.cpp) */
+#define DFQ_GEMM_FORMAT(BITS, GS, F16, NAME)                            \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 128x128, 4, 1, 1, 4, 1, 2)     \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 96x128, 3, 1, 1, 4, 1, 2)      \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128, 2, 1, 1, 4, 1, 2)      \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128_k2, 2, 1, 1, 4, 2, 2)   \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x64_k4, 1, 1, 1, 2, 4, 2)
+
+DFQ_GEMM_FORMAT(4, 32, false, bf16)
+DFQ_GEMM_FORMAT(4, 64, false, bf16)
+DFQ_GEMM_FORMAT(8, 32, false, bf16)
+DFQ_GEMM_FORMAT(8, 64, false, bf16)
+DFQ_GEMM_FORMAT(4, 32, true, f16)
+DFQ_GEMM_FORMAT(4, 64, true, f16)
+DFQ_GEMM_FORMAT(8, 32, true, f16)
+DFQ_GEMM_FORMAT(8, 64, true, f16)

@@ -129,6 +129,23 @@ typedef struct QmvParams {
     int32_t lds_out_off;    /* byte offset of the workgroup's outputs [M][rows_max] fp32 */
 } QmvParams;
 
+/* Parameters of the stock path's many-row matrix product (qmm_gemm.hip): one dtype for x,
+ * scales, biases and y. */
+typedef struct QmmGemmParams {
+    const void* x;          /* [M][K]                                                 */
+    const uint32_t* w;      /* [N][K*bits/32]                                         */
+    const void* scales;     /* [N][gpr]                                               */
+    const void* biases;     /* [N][gpr]                                               */
+    const void* lbias;      /* [N] or NULL                                            */
+    void* y;                /* [M][N]                                                 */
+    int32_t M, N, K;
+    int32_t gpr;            /* groups per row                                         */
+    int32_t gshift;         /* 1: groups of 128, taken as two of 64                   */
+    int32_t tiles_m;        /* row tiles                                              */
+    int32_t svec;           /* 1: a code line's scales (biases) are one aligned load  */
+    int32_t xcd8;           /* 1: workgroups are dealt to eight XCDs round-robin      */
+} QmmGemmParams;
+
 /* Logits per block of dfq_argmax_accept: 256 threads x DFQ_ACCEPT_CHUNK / 2048 16-byte loads
  * of 8 logits (a multiple of 2048).  Fewer, longer blocks mean fewer arrivals on the one
  * device-wide counter; measured on MI355X over [M, 151936] bf16 logits (us, M = 8 / 12 / 16):

@@ -20,8 +20,8 @@
 #include "qmm_internal.h"
 #include "qmm_params.h"
 
-#ifndef DFQ_HSACO_PATH
-#error "DFQ_HSACO_PATH must name the gfx950 code object to embed"
+#if !defined(DFQ_HSACO_PATH) || !defined(DFQ_GEMM_HSACO_PATH)
+#error "DFQ_HSACO_PATH and DFQ_GEMM_HSACO_PATH must name the gfx950 code objects to embed"
 #endif
 
 __asm__(".section .rodata.dfq_hsaco,\"a\",@progbits\n"
@@ -34,9 +34,16 @@ __asm__(".section .rodata.dfq_hsaco,\"a\",@progbits\n"
         ".hidden dfq_hsaco_end\n"
         "dfq_hsaco_end:\n"
         ".byte 0\n"
+        ".p2align 12\n"
+        ".globl dfq_gemm_hsaco_begin\n"
+        ".hidden dfq_gemm_hsaco_begin\n"
+        "dfq_gemm_hsaco_begin:\n"
+        ".incbin \"" DFQ_GEMM_HSACO_PATH "\"\n"
+        ".byte 0\n"
         ".previous\n");
 extern "C" const char dfq_hsaco_begin[];
 extern "C" const char dfq_hsaco_end[];
+extern "C" const char dfq_gemm_hsaco_begin[];
 
 namespace {
 
@@ -99,11 +106,29 @@ struct PlanKeyHash {
 
 }  // namespace
 
+/* The tiles of the stock path's many-row matrix product (qmm_gemm.hip). */
+struct GemmTile {
+    const char* name;
+    int rows, cols, threads;
+    int per_cu;   /* workgroups a CU holds (LDS) */
+    float alone;  /* us per 64 k of a workgroup that has its CU to itself */
+    float full;   /* us per 64 k and round of per_cu workgroups */
+};
+constexpr int kGemmTileCount = 5;
+static const GemmTile kGemmTiles[kGemmTileCount] = {
+    {"128x128", 128, 128, 256, 2, 1.07f, 1.57f},
+    {"96x128", 96, 128, 256, 2, 0.865f, 1.21f},
+    {"64x128", 64, 128, 256, 2, 0.665f, 0.90f},
+    {"64x128_k2", 64, 128, 512, 1, 0.556f, 0.60f},
+    {"32x64_k4", 32, 64, 512, 1, 0.273f, 0.269f},
+};
+
 struct dfq_ctx {
     int device = 0;
     int num_cus = 0;
     size_t lds_max = 0;
     hipModule_t module = nullptr;
+    hipModule_t gemm_module = nullptr;
     hipFunction_t mt8[2][3][2][2] = {};  // [bits 4/8][gs 32/64/128][bf16/f16][chunk 1/8 groups]
     hipFunction_t mt16[2][3][2] = {};    // up to 16 rows, 8-group chunks [bits][gs][bf16/f16]
     hipFunction_t am[2][3][2][2] = {};   // greedy-accept forms, 8-group chunks [..][rows 8/16]
@@ -116,6 +141,7 @@ struct dfq_ctx {
     hipFunction_t silu_mul[2] = {};      // SiLU-mul of a fused gate||up output [bf16/f16]
     hipFunction_t argmax_accept[2] = {}; // greedy accept of a verify pass [bf16/f16]
     hipFunction_t qmv[2][3][2][2] = {};  // stock-path GEMV [bits][gs][bf16/f16][rows 1 / <= 4]
+    hipFunction_t gemm[2][2][2][kGemmTileCount] = {};  // many rows [bits][gs 32/64+][bf16/f16]
     hipFunction_t generic = nullptr;
     hipFunction_t fill = nullptr;
     hipFunction_t read_stream = nullptr; // the plain streaming read (bandwidth reference)
@@ -554,6 +580,23 @@ const char* dfq_status_string(dfq_status s) {
 
 int dfq_abi_version(void) { return DFQ_ABI_VERSION; }
 
+static dfq_status load_gemm(dfq_ctx* ctx) {
+    hipError_t e = hipModuleLoadData(&ctx->gemm_module, dfq_gemm_hsaco_begin);
+    if (e != hipSuccess) return hip_fail(e, "hipModuleLoadData(gfx950 matrix-product object)");
+    for (int b = 0; b < 2; ++b)
+        for (int g = 0; g < 2; ++g)
+            for (int d = 0; d < 2; ++d)
+                for (int t = 0; t < kGemmTileCount; ++t) {
+                    char name[64];
+                    snprintf(name, sizeof name, "dfq_gemm_b%d_g%d_%s_%s", b ? 8 : 4, g ? 64 : 32,
+                             d ? "f16" : "bf16", kGemmTiles[t].name);
+                    if ((e = hipModuleGetFunction(&ctx->gemm[b][g][d][t], ctx->gemm_module,
+                                                  name)) != hipSuccess)
+                        return hip_fail(e, name);
+                }
+    return DFQ_OK;
+}
+
 dfq_status dfq_init(int device, dfq_ctx** out) {
     if (!out) return fail(DFQ_ERR_INVALID_ARGUMENT, "null out");
     *out = nullptr;
@@ -656,8 +699,10 @@ dfq_status dfq_init(int device, dfq_ctx** out) {
         delete ctx;
         return hip_fail(e, "hipModuleGetFunction");
     }
-    dfq_status st = scratch_setup(device, &ctx->scratch);
+    dfq_status st = load_gemm(ctx);
+    if (st == DFQ_OK) st = scratch_setup(device, &ctx->scratch);
     if (st != DFQ_OK) {
+        if (ctx->gemm_module) (void)hipModuleUnload(ctx->gemm_module);
         (void)hipModuleUnload(ctx->module);
         delete ctx;
         return st;
@@ -670,6 +715,7 @@ dfq_status dfq_destroy(dfq_ctx* ctx) {
     if (!ctx) return DFQ_OK;
     {
         DeviceGuard g(ctx->device);
+        if (ctx->gemm_module) (void)hipModuleUnload(ctx->gemm_module);
         if (ctx->module) (void)hipModuleUnload(ctx->module);
     }
     delete ctx;
@@ -1244,10 +1290,23 @@ dfq_status dfq_qmm_argmax_accept_packed(dfq_ctx* ctx, const void* x, const void*
                              true);
 }
 
+/* Formats and alignments both one-dtype kernels of the stock path take. */
+static bool stock_format(int bits, int gs, dfq_dtype dt, const void* x, const void* w,
+                         const void* scales, const void* biases, const void* y) {
+    return (bits == 4 || bits == 8) && (gs == 32 || gs == 64 || gs == 128) &&
+           (dt == DFQ_BF16 || dt == DFQ_F16) && aligned(x, 16) && aligned(w, 16) &&
+           aligned(scales, 2) && aligned(biases, 2) && aligned(y, 2);
+}
+
 /* Workgroups and LDS layout of the stock path's GEMV for a shape of at most 4 rows; false
  * where its x (M x K, pre-permuted, and the per-chunk sums) and outputs would not fit in LDS. */
 static constexpr int kQmvRows = 4;    // weight rows a wave works on at once (as the kernels)
 static constexpr int kQmvWaves = 8;   // waves per workgroup (as the kernels)
+/* Up to two launches of the GEMV, whose outputs depend on their own row alone, bit for bit; the
+ * matrix product takes over where a third would be due.  Measured (us, GEMV / product), K 5120:
+ * N = 5120 8 rows 25.8 / 20.4, 9 rows 34 / 20.4; N = 17408 49.2 / 41.6, 63 / 41.6; N = K = 1024
+ * 13.0 / 10.0, 16 / 10.0 (the issue of the calls). */
+static constexpr int kQmvMaxRows = 8;
 static bool qmv_layout(const dfq_ctx* ctx, int M, int N, int K, int bits, QmvParams* p,
                        size_t* lds) {
     const int kpl = 128 / bits;  // k per lane chunk
@@ -1285,9 +1344,7 @@ static bool qmv_layout(const dfq_ctx* ctx, int M, int N, int K, int bits, QmvPar
 static dfq_status qmv_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                           const void* biases, const void* lbias, void* y, int M, int N, int K,
                           int bits, int gs, dfq_dtype dt, hipStream_t stream) {
-    if ((bits != 4 && bits != 8) || (gs != 32 && gs != 64 && gs != 128) ||
-        (dt != DFQ_BF16 && dt != DFQ_F16) || !aligned(x, 16) || !aligned(w, 16) ||
-        !aligned(scales, 2) || !aligned(biases, 2) || !aligned(y, 2) ||
+    if (!stock_format(bits, gs, dt, x, w, scales, biases, y) ||
         (int64_t)N * K * bits / 8 >= (int64_t)1 << 32)
         return DFQ_ERR_UNSUPPORTED;
     QmvParams p{};
@@ -1313,6 +1370,65 @@ static dfq_status qmv_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const 
     return DFQ_OK;
 }
 
+/* The tile that finishes first by its measured step times: a CU works through its share of the
+ * tiles in rounds of per_cu workgroups, and an odd last one has the CU to itself.  Measured on
+ * MI355X (us, each tile in the table's order; the model picks the first of the best two or
+ * within 5 % of the best): 2048 x 17408, K 5120, 4-bit bf16: 535 567 612 821 1465;
+ * 512 x 5120, K 5120: 88 71 72 88 101; 200 x 17408, K 5120: 116 93 115 128 142;
+ * 333 x 5120, K 17408, 8-bit fp16: 304 248 204 188 332; 64 x 5120, K 5120: 86 69 53 45 22. */
+static int gemm_tile(int M, int N, int num_cus) {
+    int best = 0;
+    double least = 0;
+    for (int i = 0; i < kGemmTileCount; ++i) {
+        const GemmTile& t = kGemmTiles[i];
+        const int64_t tiles = (int64_t)((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
+        const int64_t share = (tiles + num_cus - 1) / num_cus;
+        const double us = (double)(share / t.per_cu) * t.full +
+                          (share % t.per_cu ? (double)t.alone : 0.0);
+        if (i == 0 || us < least) {
+            least = us;
+            best = i;
+        }
+    }
+    return best;
+}
+
+/* The stock path's matrix product for many rows (qmm_gemm.hip): one dtype of x, scales, biases
+ * and y, any M and N; DFQ_ERR_UNSUPPORTED where its loads would not be aligned or its 32-bit
+ * offsets within a tile would not hold. */
+static dfq_status gemm_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
+                           const void* biases, const void* lbias, void* y, int M, int N, int K,
+                           int bits, int gs, dfq_dtype dt, hipStream_t stream) {
+    if (!stock_format(bits, gs, dt, x, w, scales, biases, y) || K > (1 << 22))
+        return DFQ_ERR_UNSUPPORTED;
+    const int ti = gemm_tile(M, N, ctx->num_cus);
+    const GemmTile& t = kGemmTiles[ti];
+    const int gk = gs == 32 ? 32 : 64;          // the kernel's group
+    const int lg = 1024 / bits / gk;            // its groups in a 128-byte line of codes
+    const int64_t tn = (N + t.cols - 1) / t.cols, tm = (M + t.rows - 1) / t.rows;
+    if (tn * tm > INT32_MAX) return DFQ_ERR_UNSUPPORTED;
+    QmmGemmParams p{};
+    p.x = x;
+    p.w = w;
+    p.scales = scales;
+    p.biases = biases;
+    p.lbias = lbias;
+    p.y = y;
+    p.M = M;
+    p.N = N;
+    p.K = K;
+    p.gpr = K / gs;
+    p.gshift = gs == 128 ? 1 : 0;
+    p.tiles_m = (int)tm;
+    p.svec = gs != 128 && p.gpr % lg == 0 && aligned(scales, 2 * lg) && aligned(biases, 2 * lg);
+    p.xcd8 = ctx->num_cus == 256 ? 1 : 0;
+    void* args[] = {&p};
+    hipError_t e = hipModuleLaunchKernel(
+        ctx->gemm[bits == 4 ? 0 : 1][gs == 32 ? 0 : 1][dt == DFQ_BF16 ? 0 : 1][ti],
+        (unsigned)(tn * tm), 1, 1, (unsigned)t.threads, 1, 1, 0, stream, args, nullptr);
+    return e == hipSuccess ? DFQ_OK : hip_fail(e, "launch dfq_gemm");
+}
+
 dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                             const void* biases, const void* lbias, void* y, int M, int N, int K,
                             int bits, int gs, dfq_dtype xdt, dfq_dtype sdt, dfq_dtype ydt,
@@ -1333,8 +1449,13 @@ dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, cons
     if (!aligned(w, 4)) return fail(DFQ_ERR_INVALID_ARGUMENT, "w must be 4-byte aligned");
     DeviceGuard g(ctx->device);
     if (xdt == sdt && sdt == ydt) {
-        const dfq_status s = qmv_any(ctx, x, w, scales, biases, lbias, y, M, N, K, bits, gs, xdt,
-                                     (hipStream_t)stream);
+        dfq_status s = DFQ_ERR_UNSUPPORTED;
+        if (M <= kQmvMaxRows)
+            s = qmv_any(ctx, x, w, scales, biases, lbias, y, M, N, K, bits, gs, xdt,
+                        (hipStream_t)stream);
+        if (s == DFQ_ERR_UNSUPPORTED)
+            s = gemm_any(ctx, x, w, scales, biases, lbias, y, M, N, K, bits, gs, xdt,
+                         (hipStream_t)stream);
         if (s != DFQ_ERR_UNSUPPORTED) return s;
     }
     QmmGenericParams p{};
@@ -1528,14 +1649,14 @@ dfq_status dfq_debug_read_units_packed(dfq_ctx* ctx, const void* packed, int M, 
 }
 
 /* Launches of the stock path's GEMV for a shape with x, scales and y all of `dt` and 16-byte
- * aligned arrays: one per 4 rows, or 0 where the per-element path takes the call. */
+ * aligned arrays: one per 4 rows, or 0 where another kernel takes the call. */
 dfq_status dfq_debug_stock_gemv_launches(dfq_ctx* ctx, int M, int N, int K, int bits, int gs,
                                          dfq_dtype dt, int* launches) {
     if (!ctx || !launches) return fail(DFQ_ERR_INVALID_ARGUMENT, "null argument");
     QmvParams p{};
     size_t lds = 0;
     const bool ok = (bits == 4 || bits == 8) && (gs == 32 || gs == 64 || gs == 128) &&
-                    (dt == DFQ_BF16 || dt == DFQ_F16) && M >= 1 &&
+                    (dt == DFQ_BF16 || dt == DFQ_F16) && M >= 1 && M <= kQmvMaxRows &&
                     (int64_t)N * K * bits / 8 < (int64_t)1 << 32 &&
                     qmv_layout(ctx, std::min(M, 4), N, K, bits, &p, &lds);
     *launches = ok ? (M + 3) / 4 : 0;

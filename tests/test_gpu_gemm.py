@@ -1,0 +1,76 @@
+"""The stock path's many-row matrix product (dfq_qmm_fallback above 8 rows, one 16-bit dtype).
+
+Pinned two ways, in every format and at the edges of every tile:
+
+* bit-exact one-hot rows: with x[m] = e_k, power-of-two scales and small integer biases every
+  term of the factored form is exact, so y must equal the oracle's dequant bit for bit;
+* against the fp64 oracle, elementwise: the output's rounding plus the fp32 sums' bound.
+"""
+import numpy as np
+import pytest
+
+from gpu_util import announce, download, to_dev16, upload
+from onehot import exact_case
+from oracle.qmm_oracle import BF16, F16, make_case, to_bits
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [(bits, gs, dt) for bits in (4, 8) for gs in (32, 64, 128) for dt in (BF16, F16)]
+# (rows, columns) that take each tile of the dispatch on 256 CUs, with ragged edges: 32 x 64 in
+# four K slices, 64 x 128 in two, 64 x 128, 96 x 128, 128 x 128
+TILES = [(9, 37), (33, 130), (64, 16397), (193, 14001), (65, 16397), (400, 14001)]
+
+
+@pytest.mark.parametrize("bits,gs,dt", FORMATS)
+def test_one_hot_rows_are_exact(ctx, bits, gs, dt):
+    import torch
+    K = 11 * gs if gs != 128 else 5 * gs   # a ragged line, step (group 32) and slice of K
+    N = 77
+    w, sb, bb, deq = exact_case(N, K, bits, gs, dt, seed=bits * 100 + gs + dt)
+    wd = torch.from_numpy(w.view(np.int32)).cuda()
+    sd, bd = to_dev16(sb, dt), to_dev16(bb, dt)
+    x = torch.eye(K, dtype=torch.bfloat16 if dt == BF16 else torch.float16, device="cuda")
+    announce(f"stock gemm one-hot bits={bits} gs={gs} dt={dt} K={K}")
+    y = ctx.fallback(x, wd, sd, bd, bits, gs)
+    torch.cuda.synchronize()
+    got = y.view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(got, to_bits(deq.T, dt))
+
+
+@pytest.mark.parametrize("bits,gs,dt", FORMATS)
+@pytest.mark.parametrize("M,N", TILES)
+def test_matches_oracle(ctx, oracle, M, N, bits, gs, dt):
+    """|y - y64| <= u_out |y64| + (K + 8) 2^-24 S, S = sum |x| (|s| (MAGIC + q_max) + |b|): one
+    output rounding and at most K + 8 roundings of sums no larger than S (MAGIC 128 at bf16
+    4-bit, 0 otherwise), + one unit of the smallest fp16."""
+    K = {32: 352, 64: 704, 128: 640}[gs] if N < 6000 else 3 * gs
+    c = make_case(M, N, K, bits=bits, gs=gs, xdt=dt, seed=M + N + bits, lbias=(M % 2 == 1))
+    x, w, s, b, lb = upload(c)
+    announce(f"stock gemm M={M} N={N} K={K} bits={bits} gs={gs} dt={dt}")
+    y = download(ctx.fallback(x, w, s, b, bits, gs, lbias=lb))
+    ref = oracle.qmm_f64(c)
+    top = (1 << bits) - 1 + (128 if bits == 4 and dt == BF16 else 0)
+    wmax = np.repeat(np.abs(download(s)) * top + np.abs(download(b)), gs, axis=1)
+    S = np.abs(download(x)) @ wmax.T + (0 if lb is None else np.abs(download(lb)))
+    u = 2.0 ** -8 if dt == BF16 else 2.0 ** -11  # half a unit of 8 and 11 significant bits
+    bound = u * np.abs(ref) + (K + 8) * 2.0 ** -24 * S + 2.0 ** -24
+    bad = np.argwhere(~(np.abs(y - ref) <= bound))
+    assert bad.size == 0, (len(bad), bad[0], y[tuple(bad[0])], ref[tuple(bad[0])])
+
+
+def test_rows_past_the_gemvs_limit_in_k_and_misaligned_scales(ctx, oracle):
+    """K too long for the GEMV's x in LDS takes the product at any M, and scales that are not
+    aligned for a line's vector load are read one by one."""
+    import torch
+    c = make_case(3, 40, 32768, bits=4, gs=64, seed=5)
+    x, w, s, b, _ = upload(c)
+    assert ctx.stock_gemv_launches(3, 40, 32768, 4, 64) == 0
+    announce("stock gemm long K")
+    y = ctx.fallback(x, w, s, b, 4, 64)
+    buf = torch.empty(2 * s.numel() + 1, dtype=s.dtype, device="cuda")
+    s2 = buf[1:1 + s.numel()].view(s.shape).copy_(s)
+    y2 = ctx.fallback(x, w, s2, b, 4, 64)
+    torch.cuda.synchronize()
+    ref = oracle.qmm_f64(c)
+    assert np.abs(download(y) - ref).max() <= 2.0 ** -8 * np.abs(ref).max()
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
