@@ -125,6 +125,20 @@ __device__ __forceinline__ u32x4_t nibble_permute(u32x4_t v) {
     return o;
 }
 
+/* Element i of an array of dtype dt (0 bf16, 1 fp16, 2 fp32) as fp32, and the store of one. */
+__device__ __forceinline__ float load_any(const void* ptr, int dt, size_t i) {
+    if (dt == 2) return ((const float*)ptr)[i];
+    const uint16_t h = ((const uint16_t*)ptr)[i];
+    if (dt == 1) return (float)__builtin_bit_cast(_Float16, h);
+    return __uint_as_float((uint32_t)h << 16);
+}
+
+__device__ __forceinline__ void store_any(void* ptr, int dt, size_t i, float f) {
+    if (dt == 2) ((float*)ptr)[i] = f;
+    else if (dt == 1) ((uint16_t*)ptr)[i] = f32_to_out<true>(f);
+    else ((uint16_t*)ptr)[i] = f32_to_out<false>(f);
+}
+
 }  // namespace
 
 #endif

@@ -43,10 +43,9 @@
  * from sharing a CU) of 12 streaming waves, which take units of (16-column tile, chunk) from
  * an LDS counter, and one publisher wave, which writes finished tiles.
  *
- * Generic path (qmm_generic): the stock-op stand-in -- one wave per output element, plain
- * per-element dequantisation, W re-read for every row.  It exists so that the drop-in layer
- * has a fall-through for shapes outside the fast kernel's window, and so that tests can
- * prove the fast kernel really ran (its result is not bit-identical to this one).
+ * Generic path (qmm_generic): the stock-op stand-in of last resort -- one wave per output
+ * element, plain per-element dequantisation, W re-read for every row -- for the groups, lengths
+ * and alignments that neither the GEMV here nor the products of qmm_gemm.hip take.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -1475,19 +1474,6 @@ __device__ __forceinline__ void qmm_mt8(const QmmParams& p, int wg) {
 /* ---------------------------------------------------------------------------------- */
 /* Generic kernel: the stock-op stand-in                                                */
 /* ---------------------------------------------------------------------------------- */
-
-__device__ __forceinline__ float load_any(const void* ptr, int dt, size_t i) {
-    if (dt == 2) return ((const float*)ptr)[i];
-    const uint16_t h = ((const uint16_t*)ptr)[i];
-    if (dt == 1) return (float)__builtin_bit_cast(_Float16, h);
-    return __uint_as_float((uint32_t)h << 16);
-}
-
-__device__ __forceinline__ void store_any(void* ptr, int dt, size_t i, float f) {
-    if (dt == 2) ((float*)ptr)[i] = f;
-    else if (dt == 1) ((uint16_t*)ptr)[i] = f32_to_out<true>(f);
-    else ((uint16_t*)ptr)[i] = f32_to_out<false>(f);
-}
 
 /* ---------------------------------------------------------------------------------- */
 /* The stock path for few rows: a GEMV (qmv)                                            */

@@ -142,6 +142,7 @@ struct dfq_ctx {
     hipFunction_t argmax_accept[2] = {}; // greedy accept of a verify pass [bf16/f16]
     hipFunction_t qmv[2][3][2][2] = {};  // stock-path GEMV [bits][gs][bf16/f16][rows 1 / <= 4]
     hipFunction_t gemm[2][2][2][kGemmTileCount] = {};  // many rows [bits][gs 32/64+][bf16/f16]
+    hipFunction_t f32[3][2][3][3] = {};  // fp32 arithmetic [bits 2/4/8][k a lane][x dtype][rows]
     hipFunction_t generic = nullptr;
     hipFunction_t fill = nullptr;
     hipFunction_t read_stream = nullptr; // the plain streaming read (bandwidth reference)
@@ -591,6 +592,18 @@ static dfq_status load_gemm(dfq_ctx* ctx) {
                     snprintf(name, sizeof name, "dfq_gemm_b%d_g%d_%s_%s", b ? 8 : 4, g ? 64 : 32,
                              d ? "f16" : "bf16", kGemmTiles[t].name);
                     if ((e = hipModuleGetFunction(&ctx->gemm[b][g][d][t], ctx->gemm_module,
+                                                  name)) != hipSuccess)
+                        return hip_fail(e, name);
+                }
+    static const char* kXdt[3] = {"bf16", "f16", "f32"};
+    for (int b = 0; b < 3; ++b)
+        for (int k = 0; k < 2; ++k)
+            for (int d = 0; d < 3; ++d)
+                for (int r = 0; r < 3; ++r) {
+                    char name[64];
+                    snprintf(name, sizeof name, "dfq_f32_b%d_k%d_%s_r%d", 2 << b, k ? 32 : 8,
+                             kXdt[d], 1 << r);
+                    if ((e = hipModuleGetFunction(&ctx->f32[b][k][d][r], ctx->gemm_module,
                                                   name)) != hipSuccess)
                         return hip_fail(e, name);
                 }
@@ -1429,6 +1442,10 @@ static dfq_status gemm_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const
     return e == hipSuccess ? DFQ_OK : hip_fail(e, "launch dfq_gemm");
 }
 
+/* K from which a lane of the fp32 kernel takes 32 k a step rather than 8: each of the 16 waves
+ * then still has a step of 128 k. */
+static constexpr int kF32LongK = 2048;
+
 dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                             const void* biases, const void* lbias, void* y, int M, int N, int K,
                             int bits, int gs, dfq_dtype xdt, dfq_dtype sdt, dfq_dtype ydt,
@@ -1474,6 +1491,18 @@ dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, cons
     p.sdt = sdt;
     p.ydt = ydt;
     void* args[] = {&p};
+    /* fp32 arithmetic on the matrix cores where a lane's codes and x are whole aligned loads
+     * in one group; otherwise one wave per output element */
+    const size_t sal = sdt == DFQ_F32 ? 4 : 2;
+    if (K % 32 == 0 && gs % 32 == 0 && aligned(x, 16) && aligned(w, 16) && aligned(scales, sal) &&
+        aligned(biases, sal)) {
+        const int r = M <= 16 ? 0 : M <= 32 ? 1 : 2, k = K >= kF32LongK ? 1 : 0;
+        hipError_t e = hipModuleLaunchKernel(
+            ctx->f32[bits == 2 ? 0 : bits == 4 ? 1 : 2][k][(int)xdt][r], (unsigned)((N + 15) / 16),
+            (unsigned)((M + (16 << r) - 1) / (16 << r)), 1, 1024, 1, 1, 0, (hipStream_t)stream,
+            args, nullptr);
+        return e == hipSuccess ? DFQ_OK : hip_fail(e, "launch dfq_f32");
+    }
     hipError_t e = hipModuleLaunchKernel(ctx->generic, (unsigned)N, (unsigned)M, 1, 64, 1, 1, 0,
                                          (hipStream_t)stream, args, nullptr);
     return e == hipSuccess ? DFQ_OK : hip_fail(e, "launch dfq_qmm_generic");

@@ -172,8 +172,10 @@ dfq_status dfq_interleave_gate_up(dfq_ctx* ctx, const void* gate, const void* up
  * at SmallMQuantizedMatmul.swift:265), which runs a GEMV for few rows.  Where x, scales and y
  * share bf16 or fp16, bits are 4 or 8 and the group 32, 64 or 128, up to 8 rows run as that
  * GEMV where 4 rows of x fit in LDS, one launch per 4 rows (each weight row read once a launch),
- * and more rows as one matrix product on the matrix cores (its sums in another order); otherwise
- * one wave per output element, re-reading W for every row.  No workspace; asynchronous on
+ * and more rows as one matrix product on the matrix cores (its sums in another order).  Every
+ * other call has fp32 weights, products and sums: on the fp32 matrix instruction where K and the
+ * group are multiples of 32 and x and w are 16-byte aligned, else one wave per output element,
+ * re-reading W for every row.  No workspace; asynchronous on
  * `stream`. */
 dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                             const void* biases, const void* linear_bias, void* y, int M, int N,
