@@ -18,22 +18,29 @@
  *    16 k slots of one MFMA against b, and of a second against -MAGIC s (or, for fp16, the
  *    low part of b, split exactly into two bf16 values): one or two MFMAs per 16.
  *
+ *    X itself is one more product, ones . x, shared out over the column strips: summed on the
+ *    vector pipe as x is staged instead, a 128 x 128 step alone took 1.07 us against 0.83.
+ *
  * A workgroup computes 32 RT MW rows x 32 CT NW columns in KW slices of K; a wave holds RT x CT
  * tiles of one slice.  x is staged in LDS 64 k a step, in two buffers, permuted into the order
  * of the nibbles and XOR-swizzled by row so that neither writes nor reads conflict; codes are
  * staged by whole 128-byte lines of their rows (4 or 2 steps), with the line's scales and
  * biases.  Read straight into the operand registers instead, 32 bytes a row and step, the lines
  * of 128 columns and their scales outlived the 32 KB L1 and each was fetched several times:
- * 2048 x 17408, K 5120 took 556 us against 535, 16 x 5120 25.7 against 20.9.  All loads run PD
- * steps (x) or a line (codes) ahead, and are clamped rather than predicated: with a branch
+ * 2048 x 17408, K 5120 took 556 us against 535, 16 x 5120 25.7 against 20.9.  All loads run a
+ * step (x) or a line (codes) ahead, and are clamped rather than predicated: with a branch
  * around them the compiler waited for each at once (636 against 556 us).  KW > 1 slices are
  * summed through LDS at the end, in slice order.
  *
+ * The next step is staged after all but the last two row tiles' LDS reads, which its writes
+ * would otherwise hold up (2048 x 17408, K 5120: 527 us after the first, 513).
+ *
  * Measured on MI355X against the GEMV's launches it replaces (us): 512 x 5120, K 5120, 4-bit
- * bf16 1537 -> 69; 2048 x 17408, K 5120 12548 -> 535 (682 TFLOP/s); an MLP of 333 rows, 8-bit
- * fp16 6565 -> 444.  Bound by the chain of a step (staging, LDS reads, MFMAs, FMAs), which two
- * workgroups a CU overlap only in part: a wave's 64-k step of 128 x 32 needs 576 matrix cycles
- * and takes about 1600.
+ * bf16 1537 -> 58.6; 2048 x 17408, K 5120 12548 -> 517 (706 TFLOP/s); an MLP of 333 rows, 8-bit
+ * fp16 6565 -> 432.  Bound by the issue of vector instructions next to the matrix pipe: a
+ * wave's step of 128 x 32 has about 700 matrix cycles and 150 vector instructions, up to six of
+ * which issue behind an MFMA of their own wave, but another wave's only one (measured: an FMA
+ * every 32 cycles beside a wave of MFMAs), so two waves a SIMD hardly fill each other's gaps.
  */
 #include "qmm_device.h"
 #include "qmm_params.h"
@@ -88,7 +95,7 @@ __device__ __forceinline__ u32x4_t code_operand(const uint32_t* w, uint32_t mask
     return v;
 }
 
-template <int BITS, int GS, bool F16, int RT, int CT, int MW, int NW, int KW, int PD>
+template <int BITS, int GS, bool F16, int RT, int CT, int MW, int NW, int KW>
 __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
     static_assert(GS == 32 || GS == 64, "sub-groups of a step");
     constexpr int BM = 32 * RT * MW, BN = 32 * CT * NW;
@@ -105,7 +112,6 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
     constexpr bool kTwo = F16 || BITS == 4;  // a second X product
     static_assert(XI * ST == BM * 8 && WI * ST == BN * 8, "whole chunks");
     static_assert(SI * ST == 2 * BN || SI == 1, "whole rows of scales");
-    static_assert(LS % PD == 0, "a register set per step of a line");
     /* bytes of a step's x, of four groups' X, of a line of codes and of its scales + biases */
     constexpr int kA = BM * 128, kX = BM * 32, kW = BN * 128, kS = BN * LG * 4;
     constexpr int SR = LG == 2 ? 4 : 2;  // lines of scales kept: an X product may need two
@@ -150,37 +156,25 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
         xr[i] = (tl + i * ST) >> 3;
         xoff[i] = (uint32_t)min(xr[i], M - 1 - m0) * (uint32_t)K * 2u + (uint32_t)c8 * 16u;
     }
-    u32x4_t xv[PD][XI];
-    auto load_x = [&](u32x4_t (&v)[XI], int st) {
+    u32x4_t xv[XI];
+    auto load_x = [&](int st) {
         const uint32_t k0 = (uint32_t)min(first + st, steps - 1) * 64u;
         const uint8_t* src = xg + (size_t)k0 * 2;
         /* the half step a K of odd 32s ends in: chunks past it read the half before */
         const uint32_t back = (GS == 32 && k0 + (uint32_t)c8 * 8u >= (uint32_t)K) ? 64u : 0u;
 #pragma unroll
-        for (int i = 0; i < XI; ++i) v[i] = *(const u32x4_t*)(src + (xoff[i] - back));
+        for (int i = 0; i < XI; ++i) xv[i] = *(const u32x4_t*)(src + (xoff[i] - back));
     };
-    auto stage_x = [&](u32x4_t (&v)[XI], int st) {
+    auto stage_x = [&](int st) {
         const bool in = GS == 64 || (first + st) * 64 + c8 * 8 < K;
         uint8_t* ab = abuf + (st & 1) * kA;
-        uint8_t* xb = xbuf + ((st / SS) & 1) * kX;
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             if constexpr (GS == 32)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[i][e] = in ? v[i][e] : 0u;
+                for (int e = 0; e < 4; ++e) xv[i][e] = in ? xv[i][e] : 0u;
             *(u32x4_t*)(ab + xr[i] * 128 + ((c8 ^ (xr[i] & 7)) * 16)) =
-                BITS == 4 ? nibble_permute(v[i]) : v[i];
-            float X = chunk_dot<F16>(v[i], 0.0f);
-            X += dpp_f32<0xB1>(X);                             // lanes ^1
-            X += dpp_f32<0x4E>(X);                             // lanes ^2
-            if constexpr (GS == 64) X += dpp_f32<0x141>(X);    // the other half of eight
-            const uint32_t hi = __float_as_uint(X) & 0xffff0000u;
-            const float r1 = X - __uint_as_float(hi);
-            const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
-            const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
-            const int g = (NP == 1) ? (st & 3) : ((st & 1) * 2 + (c8 >> 2));
-            if ((c8 & (GS / 8 - 1)) == 0)
-                *(u32x2_t*)(xb + xr[i] * 32 + g * 8) = u32x2_t{mid | (hi >> 16), lo >> 16};
+                BITS == 4 ? nibble_permute(xv[i]) : xv[i];
         }
     };
 
@@ -264,6 +258,31 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
     __asm__ volatile("" : "+s"(nmask));  // opaque: keep in an SGPR
 
     const int line0 = first / LS;
+    /* X of one row tile's groups in step st (the strips share the row tiles): ones . x puts row
+     * l32's sum in every element of its lanes */
+    auto x_sums = [&](const uint8_t* ab, int st) {
+        const int xrow = (wm * RT + wn % RT) * 32 + l32;
+        const uint8_t* row = ab + xrow * 128;
+        uint8_t* xb = xbuf + ((st / SS) & 1) * kX + xrow * 32;
+        const u32x4_t ones = F16 ? u32x4_t{0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u}
+                                 : u32x4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            f32x16_t P = {};
+#pragma unroll
+            for (int j = 0; j < JP; ++j) {
+                const int c = (8 / NP) * q + JP * h + j;
+                P = mfma32<F16>(ones, *(const u32x4_t*)(row + ((c ^ (l32 & 7)) * 16)), P);
+            }
+            const float X = P[0];
+            const uint32_t hi = __float_as_uint(X) & 0xffff0000u;
+            const float r1 = X - __uint_as_float(hi);
+            const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
+            const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
+            const int g = (NP == 1) ? (st & 3) : ((st & 1) * 2 + q);
+            *(u32x2_t*)(xb + g * 8) = u32x2_t{mid | (hi >> 16), lo >> 16};  // (halves agree)
+        }
+    };
     /* the X products of the (up to) four groups that end with step st's */
     auto x_products = [&](int st) {
         const uint8_t* xb = xbuf + ((st / SS) & 1) * kX;
@@ -308,13 +327,12 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
         }
     };
 
-    load_x(xv[0], 0);
+    load_x(0);
     load_w(line0);
     __syncthreads();  // the zeroed X slots
-    stage_x(xv[0], 0);
+    stage_x(0);
     stage_w(line0);
-#pragma unroll
-    for (int u = 1; u <= PD; ++u) load_x(xv[u % PD], u);
+    load_x(1);
 
     for (int l = 0; l * LS < walk; ++l) {
         const int line = line0 + l;
@@ -323,12 +341,17 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
             const int st = l * LS + ls;
             if (st >= walk) break;
             __syncthreads();  // step st is staged, step st - 1 has been read
-            /* (past the end these read clamped addresses and stage what nothing reads) */
-            stage_x(xv[(ls + 1) % PD], st + 1);
-            load_x(xv[(ls + 1) % PD], st + 1 + PD);
-            if (ls == LS - 1) stage_w(line + 1);
-            if (ls == 0) load_w(line + 1);
+            if (st > 0 && ((st & (SS - 1)) == 0 || (KW > 1 && st == mine)) && st <= mine)
+                x_products(st - 1);
             if (KW > 1 && st >= mine) continue;
+            /* the next step: past the end clamped addresses are read, and what nothing reads is
+             * staged.  Placed after the LDS reads of a row tile, which it would hold up */
+            auto stage_next = [&]() {
+                stage_x(st + 1);
+                load_x(st + 2);
+                if (ls == LS - 1) stage_w(line + 1);
+                if (ls == 0) load_w(line + 1);
+            };
             const uint8_t* wb = wbuf + (line & 1) * kW;
             const uint16_t* sb = (const uint16_t*)(sbuf + (line & (SR - 1)) * kS);
             u32x4_t B[CT][4];
@@ -364,6 +387,7 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                     B[t][j] = code_operand<BITS, F16>(w + j * NWD / 4, nmask, magic);
             }
             const uint8_t* ab = abuf + (st & 1) * kA;
+            x_sums(ab, st);
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
                 const uint8_t* row = ab + ((wm * RT + r) * 32 + l32) * 128;
@@ -385,10 +409,12 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                         for (int e = 0; e < 16; ++e)
                             acc[r][t][e] = __builtin_fmaf(s[t][q], P[e], acc[r][t][e]);
                     }
+                if (r == (RT > 2 ? RT - 2 : 0)) stage_next();
             }
-            if ((st & (SS - 1)) == SS - 1 || st + 1 == mine) x_products(st);
         }
     }
+    __syncthreads();
+    if (KW == 1 || mine == walk) x_products(walk - 1);
 
     if constexpr (KW > 1) {  // the other slices' sums to slice 0
         __syncthreads();
@@ -436,18 +462,19 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
 
 }  // namespace
 
-#define DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, TILE, RT, CT, MW, NW, KW, PD)                 \
+#define DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, TILE, RT, CT, MW, NW, KW)                     \
     extern "C" __global__ void __launch_bounds__(64 * MW * NW * KW, 2)                            \
         dfq_gemm_b##BITS##_g##GS##_##NAME##_##TILE(QmmGemmParams p) {                        \
-        qmm_gemm<BITS, GS, F16, RT, CT, MW, NW, KW, PD>(p);                                      \
+        qmm_gemm<BITS, GS, F16, RT, CT, MW, NW, KW>(p);                                      \
     }
 /* rows x columns of a workgroup's tile, and slices of K (kGemmTiles in qmm_runtime.cpp) */
-#define DFQ_GEMM_FORMAT(BITS, GS, F16, NAME)                            \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 128x128, 4, 1, 1, 4, 1, 2)     \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 96x128, 3, 1, 1, 4, 1, 2)      \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128, 2, 1, 1, 4, 1, 2)      \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128_k2, 2, 1, 1, 4, 2, 2)   \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x64_k4, 1, 1, 1, 2, 4, 2)
+#define DFQ_GEMM_FORMAT(BITS, GS, F16, NAME)                         \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 128x128, 4, 1, 1, 4, 1)     \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 96x128, 3, 1, 1, 4, 1)      \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128, 2, 1, 1, 4, 1)      \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128_k2, 2, 1, 1, 4, 2)   \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x128_k2, 1, 1, 1, 4, 2)   \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x64_k4, 1, 1, 1, 2, 4)
 
 DFQ_GEMM_FORMAT(4, 32, false, bf16)
 DFQ_GEMM_FORMAT(4, 64, false, bf16)

@@ -114,13 +114,14 @@ struct GemmTile {
     float alone;  /* us per 64 k of a workgroup that has its CU to itself */
     float full;   /* us per 64 k and round of per_cu workgroups */
 };
-constexpr int kGemmTileCount = 5;
+constexpr int kGemmTileCount = 6;
 static const GemmTile kGemmTiles[kGemmTileCount] = {
-    {"128x128", 128, 128, 256, 2, 1.07f, 1.57f},
-    {"96x128", 96, 128, 256, 2, 0.865f, 1.21f},
-    {"64x128", 64, 128, 256, 2, 0.665f, 0.90f},
-    {"64x128_k2", 64, 128, 512, 1, 0.556f, 0.60f},
-    {"32x64_k4", 32, 64, 512, 1, 0.273f, 0.269f},
+    {"128x128", 128, 128, 256, 2, 0.83f, 1.52f},
+    {"96x128", 96, 128, 256, 2, 0.69f, 1.22f},
+    {"64x128", 64, 128, 256, 2, 0.59f, 0.90f},
+    {"64x128_k2", 64, 128, 512, 1, 0.50f, 0.55f},
+    {"32x128_k2", 32, 128, 512, 1, 0.396f, 0.385f},
+    {"32x64_k4", 32, 64, 512, 1, 0.249f, 0.24f},
 };
 
 struct dfq_ctx {
@@ -1385,10 +1386,10 @@ static dfq_status qmv_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const 
 
 /* The tile that finishes first by its measured step times: a CU works through its share of the
  * tiles in rounds of per_cu workgroups, and an odd last one has the CU to itself.  Measured on
- * MI355X (us, each tile in the table's order; the model picks the first of the best two or
- * within 5 % of the best): 2048 x 17408, K 5120, 4-bit bf16: 535 567 612 821 1465;
- * 512 x 5120, K 5120: 88 71 72 88 101; 200 x 17408, K 5120: 116 93 115 128 142;
- * 333 x 5120, K 17408, 8-bit fp16: 304 248 204 188 332; 64 x 5120, K 5120: 86 69 53 45 22. */
+ * MI355X (us, each tile in the table's order; the model picks the best or one within 6 % of it):
+ * 2048 x 17408, K 5120, 4-bit bf16: 513 569 644 735 1042 1220; 512 x 5120, K 5120: 68 61 70 88
+ * 102 98; 200 x 17408, K 5120: 107 89 112 118 114 131; 333 x 5120, K 17408, 8-bit fp16: 245 212
+ * 189 187 248 297; 64 x 5120, K 5120: 66 55 49 40 31 20; 16 x 17408, K 5120: 69 57 49 41 32 38. */
 static int gemm_tile(int M, int N, int num_cus) {
     int best = 0;
     double least = 0;

@@ -17,8 +17,8 @@ pytestmark = pytest.mark.gpu
 
 FORMATS = [(bits, gs, dt) for bits in (4, 8) for gs in (32, 64, 128) for dt in (BF16, F16)]
 # (rows, columns) that take each tile of the dispatch on 256 CUs, with ragged edges: 32 x 64 in
-# four K slices, 64 x 128 in two, 64 x 128, 96 x 128, 128 x 128
-TILES = [(9, 37), (33, 130), (64, 16397), (193, 14001), (65, 16397), (400, 14001)]
+# four K slices (twice), 32 x 128 and 64 x 128 in two, 64 x 128, 96 x 128, 128 x 128
+TILES = [(9, 37), (33, 130), (32, 17000), (64, 16397), (385, 9001), (65, 16397), (400, 14001)]
 
 
 @pytest.mark.parametrize("bits,gs,dt", FORMATS)
