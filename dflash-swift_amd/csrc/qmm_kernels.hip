@@ -1890,6 +1890,38 @@ __device__ __forceinline__ void silu_mul(const uint16_t* gu, uint16_t* h, int M,
         put16(h + i, silu_mul_round<F16>(g, u));
     }
 }
+/* The same for N a multiple of 8 and 16-byte aligned arrays: 16-byte pieces, n8 = N / 8 a row,
+ * one a thread.  Bound by the reads and writes of gu and h; the element form spends them two
+ * bytes a lane and a 64-bit division an element. */
+template <bool F16>
+__device__ __forceinline__ void silu_mul8(const u32x4_t* gu, u32x4_t* h, uint32_t n8,
+                                          uint32_t pieces) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= pieces) return;
+    const uint32_t m = i / n8;
+    const u32x4_t* row = gu + (size_t)m * n8 + i;  // piece i - m n8 of row m (2 n8 pieces)
+    const u32x4_t g = row[0], u = row[n8];
+    u32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t lo = silu_mul_round<F16>(elem_to_f32<F16>(g[e] & 0xffffu),
+                                                elem_to_f32<F16>(u[e] & 0xffffu));
+        const uint32_t hi = silu_mul_round<F16>(elem_to_f32<F16>(g[e] >> 16),
+                                                elem_to_f32<F16>(u[e] >> 16));
+        o[e] = lo | (hi << 16);
+    }
+    h[i] = o;
+}
+extern "C" __global__ void __launch_bounds__(256) dfq_silu_mul8_bf16(const u32x4_t* gu, u32x4_t* h,
+                                                                     uint32_t n8,
+                                                                     uint32_t pieces) {
+    silu_mul8<false>(gu, h, n8, pieces);
+}
+extern "C" __global__ void __launch_bounds__(256) dfq_silu_mul8_f16(const u32x4_t* gu, u32x4_t* h,
+                                                                    uint32_t n8,
+                                                                    uint32_t pieces) {
+    silu_mul8<true>(gu, h, n8, pieces);
+}
 extern "C" __global__ void __launch_bounds__(256) dfq_silu_mul_bf16(const uint16_t* gu,
                                                                     uint16_t* h, int M, int N) {
     silu_mul<false>(gu, h, M, N, (int64_t)blockIdx.x * 256 + threadIdx.x,

@@ -139,6 +139,7 @@ struct dfq_ctx {
     hipFunction_t c16[2][4] = {};
     hipFunction_t pack = nullptr;        // MLX arrays -> the packed layout
     hipFunction_t reduce[2] = {};        // second pass of reduce splits [bf16/f16]
+    hipFunction_t silu_mul8[2] = {};     // the same, eight neighbours a thread
     hipFunction_t silu_mul[2] = {};      // SiLU-mul of a fused gate||up output [bf16/f16]
     hipFunction_t argmax_accept[2] = {}; // greedy accept of a verify pass [bf16/f16]
     hipFunction_t qmv[2][3][2][2] = {};  // stock-path GEMV [bits][gs][bf16/f16][rows 1 / <= 4]
@@ -699,6 +700,8 @@ dfq_status dfq_init(int device, dfq_ctx** out) {
     if ((e = hipModuleGetFunction(&ctx->generic, ctx->module, "dfq_qmm_generic")) != hipSuccess ||
         (e = hipModuleGetFunction(&ctx->reduce[0], ctx->module, "dfq_qmm_reduce_bf16")) != hipSuccess ||
         (e = hipModuleGetFunction(&ctx->reduce[1], ctx->module, "dfq_qmm_reduce_f16")) != hipSuccess ||
+        (e = hipModuleGetFunction(&ctx->silu_mul8[0], ctx->module, "dfq_silu_mul8_bf16")) != hipSuccess ||
+        (e = hipModuleGetFunction(&ctx->silu_mul8[1], ctx->module, "dfq_silu_mul8_f16")) != hipSuccess ||
         (e = hipModuleGetFunction(&ctx->silu_mul[0], ctx->module, "dfq_silu_mul_bf16")) != hipSuccess ||
         (e = hipModuleGetFunction(&ctx->silu_mul[1], ctx->module, "dfq_silu_mul_f16")) != hipSuccess ||
         (e = hipModuleGetFunction(&ctx->argmax_accept[0], ctx->module, "dfq_argmax_accept_bf16")) != hipSuccess ||
@@ -1162,6 +1165,16 @@ dfq_status dfq_silu_mul(dfq_ctx* ctx, const void* gu, void* h, int M, int N, dfq
         return fail(DFQ_ERR_INVALID_ARGUMENT, "gu and h must be 2-byte aligned");
     DeviceGuard g(ctx->device);
     const uint64_t total = (uint64_t)M * N;
+    /* eight neighbours a thread where rows are whole 16-byte pieces (and a piece's index is 32
+     * bits), one element otherwise: 333 x 17408 fp16 11.7 -> 7.5 us. */
+    if (N % 8 == 0 && aligned(gu, 16) && aligned(h, 16) && total / 8 <= INT32_MAX) {
+        uint32_t n8 = (uint32_t)N / 8, pieces = (uint32_t)(total / 8);
+        void* vargs[] = {(void*)&gu, &h, &n8, &pieces};
+        hipError_t e = hipModuleLaunchKernel(ctx->silu_mul8[dtype == DFQ_BF16 ? 0 : 1],
+                                             (pieces + 255) / 256, 1, 1, 256, 1, 1, 0,
+                                             (hipStream_t)stream, vargs, nullptr);
+        return e == hipSuccess ? DFQ_OK : hip_fail(e, "launch dfq_silu_mul8");
+    }
     unsigned grid = (unsigned)std::min<uint64_t>((total + 255) / 256, 8192);
     void* args[] = {(void*)&gu, &h, &M, &N};
     hipError_t e = hipModuleLaunchKernel(ctx->silu_mul[dtype == DFQ_BF16 ? 0 : 1], grid, 1, 1,

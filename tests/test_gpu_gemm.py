@@ -74,3 +74,19 @@ def test_rows_past_the_gemvs_limit_in_k_and_misaligned_scales(ctx, oracle):
     ref = oracle.qmm_f64(c)
     assert np.abs(download(y) - ref).max() <= 2.0 ** -8 * np.abs(ref).max()
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N", [(1, 8), (3, 1000), (257, 24), (333, 4096)])
+def test_silu_mul_by_pieces_equals_by_elements(ctx, M, N, dt):
+    """Rows of whole 16-byte pieces go eight elements a thread; arrays two bytes off that
+    alignment go one by one: the same values, bit for bit."""
+    import torch
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float16
+    buf = torch.randn(2 * M * N + 1, device="cuda", dtype=torch.float32).mul_(3).to(tdt)
+    odd = buf[1:].view(M, 2 * N)
+    announce(f"silu_mul pieces {dt} M={M} N={N}")
+    h = ctx.silu_mul(odd.clone())
+    h_odd = ctx.silu_mul(odd)
+    torch.cuda.synchronize()
+    assert torch.equal(h.view(torch.int16), h_odd.view(torch.int16))
