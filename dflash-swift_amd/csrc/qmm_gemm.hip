@@ -275,8 +275,12 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                 P = mfma32<F16>(ones, *(const u32x4_t*)(row + ((c ^ (l32 & 7)) * 16)), P);
             }
             const float X = P[0];
-            const uint32_t hi = __float_as_uint(X) & 0xffff0000u;
-            const float r1 = X - __uint_as_float(hi);
+            /* an infinite X keeps its sign: no low parts, and (fp16, whose low part of b is
+             * mostly 0) the largest finite value, so that s P decides */
+            const bool inf = __builtin_fabsf(X) == __builtin_inff();
+            uint32_t hi = __float_as_uint(X) & 0xffff0000u;
+            if (F16 && inf) hi = (hi & 0x80000000u) | 0x7f7f0000u;
+            const float r1 = inf ? 0.0f : X - __uint_as_float(hi);
             const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
             const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
             const int g = (NP == 1) ? (st & 3) : ((st & 1) * 2 + q);

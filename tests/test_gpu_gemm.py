@@ -76,6 +76,24 @@ def test_rows_past_the_gemvs_limit_in_k_and_misaligned_scales(ctx, oracle):
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
+@pytest.mark.parametrize("dt", [BF16, F16])
+def test_an_infinite_activation_stays_in_its_row(ctx, dt):
+    """8-bit codes and biases above zero: the row with the infinity is infinite, as the fp64
+    product has it, and no other row changes."""
+    import torch
+    c = make_case(20, 40, 512, bits=8, gs=64, xdt=dt, seed=2)
+    x, w, s, b, _ = upload(c)
+    b, w = b.abs() + 0.5, w | 0x01010101  # (a code of 0 times infinity is NaN)
+    announce(f"stock gemm infinity dt={dt}")
+    want = ctx.fallback(x, w, s, b, 8, 64)
+    x[7, 100] = float("inf")
+    y = ctx.fallback(x, w, s, b, 8, 64)
+    torch.cuda.synchronize()
+    keep = [r for r in range(20) if r != 7]
+    assert torch.equal(y[keep].view(torch.int16), want[keep].view(torch.int16))
+    assert (y[7] == float("inf")).all()
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("M,N", [(1, 8), (3, 1000), (257, 24), (333, 4096)])
 def test_silu_mul_by_pieces_equals_by_elements(ctx, M, N, dt):
