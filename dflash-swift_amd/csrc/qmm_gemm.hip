@@ -16,7 +16,7 @@
  *  - the X terms are a product over groups, so they go through the matrix cores too: X is
  *    split exactly into three bf16 values (24 bits), and 4 groups x (Xh, Xm, Xl, 0) are the
  *    16 k slots of one MFMA against b, and of a second against -MAGIC s (or, for fp16, the
- *    low part of b, split exactly into two bf16 values): one or two MFMAs per 16.
+ *    second part of b, split exactly into two bf16 values): one or two MFMAs per 16.
  *
  *    X itself is one more product, ones . x, shared out over the column strips: summed on the
  *    vector pipe as x is staged instead, a 128 x 128 step alone took 1.07 us against 0.83.
@@ -275,11 +275,9 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                 P = mfma32<F16>(ones, *(const u32x4_t*)(row + ((c ^ (l32 & 7)) * 16)), P);
             }
             const float X = P[0];
-            /* an infinite X keeps its sign: no low parts, and (fp16, whose low part of b is
-             * mostly 0) the largest finite value, so that s P decides */
+            /* an infinite X has no low parts (inf - inf) and stays an infinity */
             const bool inf = __builtin_fabsf(X) == __builtin_inff();
-            uint32_t hi = __float_as_uint(X) & 0xffff0000u;
-            if (F16 && inf) hi = (hi & 0x80000000u) | 0x7f7f0000u;
+            const uint32_t hi = __float_as_uint(X) & 0xffff0000u;
             const float r1 = inf ? 0.0f : X - __uint_as_float(hi);
             const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
             const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
@@ -305,10 +303,15 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                 const uint32_t cs = in ? sl[0] : 0u, cb = in ? sl[BN * LG] : 0u;
                 uint32_t v1, v2;  // the bf16 factors, in the low half
                 if constexpr (F16) {
+                    /* the low part of a short b would be 0, and NaN against an infinite X: two
+                     * halves, so that b X has the sign of both (or is NaN for b = 0, as the
+                     * GEMV's is) and s P of the other sign makes NaN, not its own infinity */
                     const float b = elem_to_f32<true>(cb);
-                    const uint32_t bh = __float_as_uint(b) & 0xffff0000u;
-                    v1 = bh >> 16;
-                    v2 = __float_as_uint(b - __uint_as_float(bh)) >> 16;
+                    const uint32_t top = __float_as_uint(b) & 0xffff0000u;
+                    const bool whole = __uint_as_float(top) == b;
+                    const float hi = whole ? 0.5f * b : __uint_as_float(top);
+                    v1 = __float_as_uint(hi) >> 16;
+                    v2 = __float_as_uint(whole ? hi : b - hi) >> 16;
                 } else {
                     v1 = cb;
                     v2 = __float_as_uint(-128.0f * elem_to_f32<false>(cs)) >> 16;

@@ -11,7 +11,7 @@ import pytest
 
 from gpu_util import announce, download, to_dev16, upload
 from onehot import exact_case
-from oracle.qmm_oracle import BF16, F16, make_case, to_bits
+from oracle.qmm_oracle import BF16, F16, make_case, pack, to_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -92,6 +92,49 @@ def test_an_infinite_activation_stays_in_its_row(ctx, dt):
     keep = [r for r in range(20) if r != 7]
     assert torch.equal(y[keep].view(torch.int16), want[keep].view(torch.int16))
     assert (y[7] == float("inf")).all()
+
+
+def classes_case(M, N, K, bits, gs, dt, seed, positive=False):
+    """MLX-style weights: s > 0 and b the group's minimum, below zero (above it and no code of 0
+    if `positive`); returns tensors and the dequantised weight."""
+    import torch
+    rng = np.random.default_rng(seed)
+    tdt = torch.bfloat16 if dt == BF16 else torch.float16
+    top = (1 << bits) - 1
+    codes = rng.integers(1 if positive else 0, top + 1, size=(N, K), dtype=np.uint8)
+    t = lambda a: torch.from_numpy(a.astype(np.float32)).to(tdt).cuda()
+    s = t(rng.uniform(0.5, 1.5, size=(N, K // gs)) / top)
+    b = t(rng.uniform(0.3, 0.7, size=(N, K // gs)) * (1 if positive else -1))
+    x = t(rng.normal(size=(M, K)))
+    w = torch.from_numpy(pack(codes, bits).view(np.int32)).cuda()
+    rep = lambda a: np.repeat(a.double().cpu().numpy(), gs, axis=1)
+    return x, w, s, b, codes * rep(s) + rep(b)
+
+
+@pytest.mark.parametrize("bits,gs,dt", FORMATS)
+def test_an_infinite_activation_never_gives_the_wrong_sign(ctx, bits, gs, dt):
+    """Biases below zero, as quantised weights have: s P and b X are infinities of either sign, so
+    the factored form gives NaN where the weight's sign cannot be told, as the GEMV does, and
+    never an infinity that the weight does not give."""
+    import torch
+    K = 11 * gs if gs != 128 else 5 * gs
+    x, w, s, b, deq = classes_case(20, 70, K, bits, gs, dt, seed=bits + gs)
+    announce(f"stock gemm infinity, negative biases bits={bits} gs={gs} dt={dt}")
+    want = ctx.fallback(x, w, s, b, bits, gs)
+    hit = {5: (3, 1.0), 7: (gs + 1, -1.0), 11: (K - 1, 1.0)}
+    for m, (k, sign) in hit.items():
+        x[m, k] = sign * float("inf")
+    y = ctx.fallback(x, w, s, b, bits, gs)
+    gemv = ctx.fallback(x[4:12].contiguous(), w, s, b, bits, gs)
+    torch.cuda.synchronize()
+    keep = [r for r in range(20) if r not in hit]
+    assert torch.equal(y[keep].view(torch.int16), want[keep].view(torch.int16))
+    for m, (k, sign) in hit.items():
+        got, few = download(y[m:m + 1])[0], download(gemv[m - 4:m - 3])[0]
+        right = np.sign(deq[:, k]) * sign * np.inf
+        assert not np.isfinite(got).any()
+        assert (np.isnan(got) | (got == right)).all()
+        assert (np.isnan(few) | ~np.isnan(got)).all()  # no NaN where the GEMV has none
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
