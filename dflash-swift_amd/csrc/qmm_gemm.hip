@@ -144,7 +144,6 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
     uint8_t* xbuf = abuf + 2 * kA;
     uint8_t* wbuf = xbuf + 2 * kX;
     uint8_t* sbuf = wbuf + 2 * kW;
-    for (int i = tl; i < 2 * kX / 4; i += ST) ((uint32_t*)xbuf)[i] = 0;  // unused slots
     const int c8 = tl & 7;
 
     /* x: chunk c of row r of the tile, rows past M read the last one */
@@ -336,7 +335,6 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
 
     load_x(0);
     load_w(line0);
-    __syncthreads();  // the zeroed X slots
     stage_x(0);
     stage_w(line0);
     load_x(1);
@@ -348,8 +346,7 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
             const int st = l * LS + ls;
             if (st >= walk) break;
             __syncthreads();  // step st is staged, step st - 1 has been read
-            if (st > 0 && ((st & (SS - 1)) == 0 || (KW > 1 && st == mine)) && st <= mine)
-                x_products(st - 1);
+            if (st > 0 && (st & (SS - 1)) == 0 && st <= mine) x_products(st - 1);
             if (KW > 1 && st >= mine) continue;
             /* the next step: past the end clamped addresses are read, and what nothing reads is
              * staged.  Placed after the LDS reads of a row tile, which it would hold up */
@@ -420,8 +417,15 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
             }
         }
     }
+    /* the last set's slots past the slice's last step: the sums of two sets before are still
+     * there (or nothing yet), and an infinity among them would make NaN of the factor 0 */
+    const int over = mine > 0 ? mine & (SS - 1) : 0;
+    if (over) {
+        uint8_t* xb = xbuf + ((mine / SS) & 1) * kX + ((wm * RT + wn % RT) * 32 + l32) * 32;
+        for (int g = over * NP; g < 4; ++g) *(u32x2_t*)(xb + g * 8) = u32x2_t{0u, 0u};
+    }
     __syncthreads();
-    if (KW == 1 || mine == walk) x_products(walk - 1);
+    if (over || mine == walk) x_products(mine - 1);
 
     if constexpr (KW > 1) {  // the other slices' sums to slice 0
         __syncthreads();

@@ -137,6 +137,21 @@ def test_an_infinite_activation_never_gives_the_wrong_sign(ctx, bits, gs, dt):
         assert (np.isnan(few) | ~np.isnan(got)).all()  # no NaN where the GEMV has none
 
 
+@pytest.mark.parametrize("bits,gs,dt", [f for f in FORMATS if f[0] == 8 or f[2] == F16])
+@pytest.mark.parametrize("M,N", [(47, 40), (47, 17000), (400, 9001)])
+def test_an_infinity_stays_one_in_every_group(ctx, M, N, bits, gs, dt):
+    """Weights above zero, an infinity in each row at another place: every output is +inf, also
+    where the last groups of a slice of K are fewer than an X product takes."""
+    import torch
+    K = 2944 if gs == 128 else 3008  # 46 or 47 steps of 64 k
+    x, w, s, b, _ = classes_case(M, N, K, bits, gs, dt, seed=M + gs, positive=True)
+    x[torch.arange(M), (torch.arange(M) * (64 if M < 64 else 8) + 5) % K] = float("inf")
+    announce(f"stock gemm infinity by group M={M} N={N} bits={bits} gs={gs} dt={dt}")
+    y = ctx.fallback(x, w, s, b, bits, gs)
+    bad = (y != float("inf")).nonzero().cpu()
+    assert len(bad) == 0, (len(bad), bad[0])
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("M,N", [(1, 8), (3, 1000), (257, 24), (333, 4096)])
 def test_silu_mul_by_pieces_equals_by_elements(ctx, M, N, dt):
