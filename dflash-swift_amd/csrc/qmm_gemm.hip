@@ -315,10 +315,13 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                     v1 = cb;
                     v2 = __float_as_uint(-128.0f * elem_to_f32<false>(cs)) >> 16;
                 }
-                b1[t][2 * e] = v1 | (v1 << 16);
-                b1[t][2 * e + 1] = v1;
-                b2[t][2 * e] = v2 | (v2 << 16);
-                b2[t][2 * e + 1] = v2;
+                /* an infinite b meets X's high part alone: the low ones may be 0 */
+                const bool finite = (v1 & 0x7f80u) != 0x7f80u;
+                const uint32_t l1 = finite ? v1 : 0u, l2 = !F16 || finite ? v2 : 0u;
+                b1[t][2 * e] = v1 | (l1 << 16);
+                b1[t][2 * e + 1] = l1;
+                b2[t][2 * e] = v2 | (l2 << 16);
+                b2[t][2 * e + 1] = l2;
             }
         }
 #pragma unroll

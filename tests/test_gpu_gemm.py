@@ -152,6 +152,29 @@ def test_an_infinity_stays_one_in_every_group(ctx, M, N, bits, gs, dt):
     assert len(bad) == 0, (len(bad), bad[0])
 
 
+@pytest.mark.parametrize("bits,gs,dt", FORMATS)
+def test_an_infinite_bias_gives_infinities(ctx, bits, gs, dt):
+    """Positive activations whose group sums are short numbers (no low parts): the column of an
+    infinite bias is infinite, as the GEMV has it, and no other column changes."""
+    import torch
+    K = 11 * gs if gs != 128 else 5 * gs
+    x, w, s, b, _ = classes_case(20, 70, K, bits, gs, dt, seed=bits + gs)
+    x.fill_(0.5)
+    announce(f"stock gemm infinite bias bits={bits} gs={gs} dt={dt}")
+    want = ctx.fallback(x, w, s, b, bits, gs)
+    hit = {3: (0, 1.0), 40: (K // gs - 1, -1.0), 69: (2, 1.0)}
+    for n, (g, sign) in hit.items():
+        b[n, g] = sign * float("inf")
+    y = ctx.fallback(x, w, s, b, bits, gs)
+    gemv = ctx.fallback(x[:8].contiguous(), w, s, b, bits, gs)
+    torch.cuda.synchronize()
+    keep = [n for n in range(70) if n not in hit]
+    assert torch.equal(y[:, keep].view(torch.int16), want[:, keep].view(torch.int16))
+    for n, (_, sign) in hit.items():
+        assert (gemv[:, n] == sign * float("inf")).all()
+        assert (y[:, n] == sign * float("inf")).all(), n
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("M,N", [(1, 8), (3, 1000), (257, 24), (333, 4096)])
 def test_silu_mul_by_pieces_equals_by_elements(ctx, M, N, dt):
