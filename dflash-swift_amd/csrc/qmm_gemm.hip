@@ -3,11 +3,19 @@
  * below, many rows of one 16-bit dtype of x, scales, biases and y; at the end of the file, the
  * fp32 form of every other call.
  *
- * The codes enter the MFMAs as exact small integers and everything else stays in fp32, as in
- * the GEMV: per quantisation group P = sum x (MAGIC + q), y += s * P + b * X - MAGIC * s * X
- * with X = sum x.  bf16 4-bit codes carry MAGIC = 128 (7 VALU operations make the 8 operands
- * of a word); fp16 codes take one packed subtraction more and carry none; 8-bit bf16 codes
- * are converted.
+ * The codes enter the MFMAs as exact small integers and everything else stays in fp32: per
+ * quantisation group P = sum x (MAGIC + q), y += s * P + b * X - MAGIC * s * X with X = sum x.
+ * bf16 4-bit codes carry MAGIC = 16 (8 VALU operations make the 8 operands of a word); fp16 codes
+ * take one packed subtraction more and carry none; 8-bit bf16 codes are converted.
+ *
+ *  - Precision.  The GEMV corrects each lane's 32 or 16 k at once, in 64 chains; here one
+ *    accumulator holds up to four groups' s P before the X terms meet them.  The error of the
+ *    sums before the output's rounding, as a share of the result's norm, K = 1024 to 17408,
+ *    activations of either sign / of one sign (GEMV in brackets): 4-bit bf16 1.8e-7 to 3.2e-7 /
+ *    1.9e-6 to 3.0e-6 (7.4e-7 to 8.3e-7 / 3.9e-6 to 4.1e-6; with a MAGIC of 128 here 1.4e-6 to
+ *    1.7e-6 / 1.3e-5 to 2.0e-5); 4-bit fp16 1.0e-7 to 3.2e-7 / 6.7e-7 to 1.9e-6 (1.4e-5 /
+ *    6.4e-5); 8-bit 0.9e-7 to 3.4e-7 / 0.6e-6 to 2.8e-6 (0.4e-7 to 1.4e-7 / 1.0e-7 to 2.8e-7).
+ *    The output's own rounding is 1.7e-3 in bf16 and 2.1e-4 in fp16.
  *
  *  - s * P is one fp32 FMA an accumulator element and group: 64 issue cycles a 32 x 32 tile
  *    against 128 matrix cycles at group 64, so the vector and the matrix pipes run side by
@@ -61,6 +69,24 @@ __device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
                                                        0);
 }
 
+/* 8 nibbles of a word -> bf16 (MAGIC + q) pairs (q_i, q_{i+4}) with MAGIC = 16: each code right
+ * below the leading one.  One operation more than nibble_operand's 128 + q: there the sums are
+ * 128 sum x too large until the X terms meet them, which in a long-lived accumulator costs
+ * precision (see the head comment).  TURNED words have been turned left by 3 bits as they were
+ * staged, which takes the operation out of the step's chain: 512 x 5120, K 5120 59.7 us against
+ * 61.4; with four row tiles a wave the registers of it spill (2048 x 17408 540 us against 531,
+ * with the 128 of before 525). */
+constexpr int kMagic = 16;
+template <bool TURNED>
+__device__ __forceinline__ u32x4_t nibble_operand16(uint32_t p, uint32_t mask, uint32_t magic) {
+    u32x4_t v;
+    v[0] = ((TURNED ? p : p << 3) & mask) | magic;
+    v[1] = ((p >> (TURNED ? 4 : 1)) & mask) | magic;
+    v[2] = ((p >> (TURNED ? 8 : 5)) & mask) | magic;
+    v[3] = ((TURNED ? __builtin_amdgcn_alignbit(p, p, 12) : p >> 9) & mask) | magic;
+    return v;
+}
+
 /* (1024 + q) pairs -> q pairs, exact. */
 __device__ __forceinline__ uint32_t less_1024(uint32_t v) {
     const f16x2_t m = {(_Float16)1024.0f, (_Float16)1024.0f};
@@ -75,12 +101,13 @@ __device__ __forceinline__ uint16_t round_out(float f) {
 }
 
 /* The operand of one word of 4-bit codes, or of two words of 8-bit codes. */
-template <int BITS, bool F16>
+template <int BITS, bool F16, bool TURNED>
 __device__ __forceinline__ u32x4_t code_operand(const uint32_t* w, uint32_t mask,
                                                 uint32_t magic) {
     u32x4_t v;
     if constexpr (BITS == 4) {
-        v = nibble_operand<F16>(w[0], mask, magic);
+        if constexpr (F16) v = nibble_operand<true>(w[0], mask, magic);
+        else v = nibble_operand16<TURNED>(w[0], mask, magic);
     } else if constexpr (F16) {
         v[0] = __builtin_amdgcn_perm(0x64646464u, w[0], 0x04010400u);
         v[1] = __builtin_amdgcn_perm(0x64646464u, w[0], 0x04030402u);
@@ -110,6 +137,7 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
     constexpr int WI = BN * 8 / ST;     // 16-byte chunks of codes, a line
     constexpr int SI = 2 * BN > ST ? 2 * BN / ST : 1;  // columns' scales or biases, a line
     constexpr bool kTwo = F16 || BITS == 4;  // a second X product
+    constexpr bool kTurned = BITS == 4 && !F16 && RT < 4;  // see nibble_operand16
     static_assert(XI * ST == BM * 8 && WI * ST == BN * 8, "whole chunks");
     static_assert(SI * ST == 2 * BN || SI == 1, "whole rows of scales");
     /* bytes of a step's x, of four groups' X, of a line of codes and of its scales + biases */
@@ -234,6 +262,10 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
 #pragma unroll
         for (int i = 0; i < WI; ++i) {
             const int r = (tl + i * ST) >> 3;
+            if constexpr (kTurned)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    wv[i][e] = __builtin_amdgcn_alignbit(wv[i][e], wv[i][e], 29);
             *(u32x4_t*)(wb + r * 128 + ((c8 ^ (r & 7)) * 16)) = wv[i];
         }
         uint32_t* sb = (uint32_t*)(sbuf + (line & (SR - 1)) * kS);
@@ -251,8 +283,8 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
         for (int r = 0; r < RT; ++r)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[r][t][e] = 0.0f;
-    uint32_t magic = F16 ? 0x64006400u : 0x43004300u;
-    uint32_t nmask = 0x000F000Fu;
+    uint32_t magic = F16 ? 0x64006400u : 0x41804180u;
+    uint32_t nmask = F16 ? 0x000F000Fu : 0x00780078u;
     __asm__ volatile("" : "+v"(magic));  // opaque: keep in a VGPR (see nibble_operand)
     __asm__ volatile("" : "+s"(nmask));  // opaque: keep in an SGPR
 
@@ -313,7 +345,7 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                     v2 = __float_as_uint(whole ? hi : b - hi) >> 16;
                 } else {
                     v1 = cb;
-                    v2 = __float_as_uint(-128.0f * elem_to_f32<false>(cs)) >> 16;
+                    v2 = __float_as_uint(-(float)kMagic * elem_to_f32<false>(cs)) >> 16;
                 }
                 /* an infinite b meets X's high part alone: the low ones may be 0 */
                 const bool finite = (v1 & 0x7f80u) != 0x7f80u;
@@ -391,7 +423,7 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
                 }
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    B[t][j] = code_operand<BITS, F16>(w + j * NWD / 4, nmask, magic);
+                    B[t][j] = code_operand<BITS, F16, kTurned>(w + j * NWD / 4, nmask, magic);
             }
             const uint8_t* ab = abuf + (st & 1) * kA;
             x_sums(ab, st);

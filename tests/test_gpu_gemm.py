@@ -76,6 +76,36 @@ def test_rows_past_the_gemvs_limit_in_k_and_misaligned_scales(ctx, oracle):
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("one_sign", [False, True])
+def test_four_bit_sums_are_no_further_off_than_the_gemvs(ctx, gs, dt, one_sign):
+    """Sums that are exactly 0, so that the output's rounding does not hide theirs: every group of
+    x meets codes q with bias -j s and codes 15 - q with bias -(15 - j) s, in shuffled order.  The
+    outputs are the sums' own errors, and the matrix product's are no larger (root mean square)
+    than the GEMV's on the same inputs, in a tile of four slices of K and in one of none."""
+    import torch
+    K, rng = 2560, np.random.default_rng(gs + dt)
+    G, tdt = K // gs, torch.bfloat16 if dt == BF16 else torch.float16
+    for M, N in ((16, 300), (400, 14001)):
+        q = rng.integers(0, 16, size=(N, G // 2, gs), dtype=np.uint8)
+        s = rng.integers(8, 16, size=(N, G // 2)) * 2.0 ** -13
+        j = rng.integers(5, 11, size=(N, G // 2))  # (four bits by four: exact in either dtype)
+        x = rng.normal(size=(M, G // 2, gs))
+        perm = rng.permutation(G)
+        twice = lambda a, b: np.concatenate([a, b], 1)[:, perm]
+        t = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(tdt).cuda()
+        w = pack(twice(q, 15 - q).reshape(N, K), 4)
+        w = torch.from_numpy(w.view(np.int32)).cuda()
+        sd, bd = t(twice(s, s)), t(twice(-s * j, -s * (15 - j)))
+        xd = t(twice(np.abs(x) if one_sign else x, np.abs(x) if one_sign else x).reshape(M, K))
+        announce(f"stock gemm precision gs={gs} dt={dt} one_sign={one_sign} M={M}")
+        rms = lambda y: y.double().pow(2).mean().sqrt().item()
+        got = rms(ctx.fallback(xd, w, sd, bd, 4, gs))
+        gemv = rms(ctx.fallback(xd[:8].contiguous(), w, sd, bd, 4, gs))
+        assert 0 < got <= gemv, (M, got / gemv)
+
+
 @pytest.mark.parametrize("dt", [BF16, F16])
 def test_an_infinite_activation_stays_in_its_row(ctx, dt):
     """8-bit codes and biases above zero: the row with the infinity is infinite, as the fp64
