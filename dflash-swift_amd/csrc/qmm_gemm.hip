@@ -555,6 +555,16 @@ __device__ __forceinline__ void codes8(const uint32_t* w, float (&q)[8]) {
     }
 }
 
+/* Element i of an array of dtype dt as loaded, and its value: apart, so that the loads of a step
+ * are in flight together (a conversion in the branch on dt would wait for its own). */
+__device__ __forceinline__ uint32_t load_bits(const void* ptr, int dt, size_t i) {
+    if (dt == 2) return ((const uint32_t*)ptr)[i];
+    return ((const uint16_t*)ptr)[i];
+}
+__device__ __forceinline__ float bits_to_f32(uint32_t v, int dt) {
+    return dt == 2 ? __uint_as_float(v) : dt == 1 ? elem_to_f32<true>(v) : elem_to_f32<false>(v);
+}
+
 /* y = x . dequant(W)^T with every weight, product and sum in fp32: w = s q + b is formed in
  * fp32 as the per-element kernel forms it, and the products run on the fp32 matrix
  * instruction (16 x 16 x 4), which needs x and w unsplit.
@@ -566,14 +576,18 @@ __device__ __forceinline__ void codes8(const uint32_t* w, float (&q)[8]) {
  * (t mod 4): 64 chains in a workgroup, as the per-element kernel's lanes, which keeps the
  * rounding error where it was.  The waves' sums meet in LDS and are added as a tree.
  *
+ * With one row tile the loads of two of a wave's steps are issued together (more tiles would
+ * spill): 16 x 16, K 17408, all fp32 58.7 -> 48.7 us.
+ *
  * Measured on MI355X, fp32 x over bf16 scales, 6 x 4096, K 4096, 4-bit: 172.4 us by the
- * per-element kernel, 12.6 here, most of it the issue of the call; both are 1.6e-7 from the
- * 64-bit result.  Bound by latency: a wave has two steps, each one round of loads. */
+ * per-element kernel, 12.6 a pass here; both are 1.6e-7 from the 64-bit result.  Bound by latency: a wave
+ * has two steps. */
 template <int BITS, int KL, int XDT, int RT>
 __device__ __forceinline__ void qmm_f32(const QmmGenericParams& p) {
     __shared__ f32x4_t part[kF32Waves * RT * 64];
     constexpr int CB = KL * BITS / 8;  // bytes of a lane's codes
     constexpr int XB = XDT == 2 ? 4 : 2;
+    constexpr int U = RT == 1 ? 2 : 1;  // steps whose loads are issued together
     const int tid = threadIdx.x, lane = tid & 63, n16 = lane & 15, j = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = p.M, N = p.N, K = p.K;
@@ -592,66 +606,86 @@ __device__ __forceinline__ void qmm_f32(const QmmGenericParams& p) {
 #pragma unroll
         for (int a = 0; a < 4; ++a) acc[r][a] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const int steps = (K + 4 * KL - 1) / (4 * KL);
-    for (int st = wave; st < steps; st += kF32Waves) {
+    constexpr int XW = XDT == 2 ? KL / 4 : KL / 8;  // 16-byte loads of a lane's x of one row
+    constexpr int WD = CB < 4 ? 1 : CB / 4;         // words of its codes
+    struct Step {
+        uint32_t w[WD];
+        u32x4_t x[U > 1 ? XW : 1];  // the one row tile's (more of them would spill)
+        uint32_t s, b;  // as loaded
+        int kc;
+        bool in;
+    };
+    auto load_x = [&](int r, int i, int kc) {
+        return *(const u32x4_t*)(xr[r] + (size_t)kc * XB + i * 16);
+    };
+    auto load = [&](int st) {
+        Step v;
         const int k = st * 4 * KL + j * KL;
         const bool in = k < K;  // (K is a multiple of KL) lanes past K read its last codes
         const int kc = in ? k : K - KL;
-        uint32_t w[CB < 4 ? 1 : CB / 4];
         const uint8_t* ws = wr + (size_t)kc * BITS / 8;
         if constexpr (CB == 2) {
-            w[0] = *(const uint16_t*)ws;
+            v.w[0] = *(const uint16_t*)ws;
         } else if constexpr (CB == 4) {
-            w[0] = *(const uint32_t*)ws;
+            v.w[0] = *(const uint32_t*)ws;
         } else if constexpr (CB == 8) {
-            const u32x2_t v = *(const u32x2_t*)ws;
-            w[0] = v[0];
-            w[1] = v[1];
+            const u32x2_t c = *(const u32x2_t*)ws;
+            v.w[0] = c[0];
+            v.w[1] = c[1];
         } else {
 #pragma unroll
             for (int i = 0; i < CB / 16; ++i) {
-                const u32x4_t v = *(const u32x4_t*)(ws + i * 16);
+                const u32x4_t c = *(const u32x4_t*)(ws + i * 16);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w[i * 4 + e] = v[e];
+                for (int e = 0; e < 4; ++e) v.w[i * 4 + e] = c[e];
             }
         }
         const size_t g = (size_t)n * gpr + kc / p.gs;
-        const float s = in ? load_any(p.scales, p.sdt, g) : 0.0f;
-        const float b = in ? load_any(p.biases, p.sdt, g) : 0.0f;
+        v.s = load_bits(p.scales, p.sdt, g);
+        v.b = load_bits(p.biases, p.sdt, g);
+        v.kc = kc;
+        v.in = in;
+        if constexpr (U > 1)
+#pragma unroll
+            for (int i = 0; i < XW; ++i) v.x[i] = load_x(0, i, kc);
+        return v;
+    };
+    auto add = [&](const Step& v) {
+        const float s = v.in ? bits_to_f32(v.s, p.sdt) : 0.0f;
+        const float b = v.in ? bits_to_f32(v.b, p.sdt) : 0.0f;
 #pragma unroll
         for (int c = 0; c < KL / 8; ++c) {
             float q[8];
             uint32_t wc[2];
             if constexpr (BITS == 8) {
-                wc[0] = w[2 * c];
-                wc[1] = w[2 * c + 1];
+                wc[0] = v.w[2 * c];
+                wc[1] = v.w[2 * c + 1];
             } else if constexpr (BITS == 4) {
-                wc[0] = w[c];
+                wc[0] = v.w[c];
             } else {
-                wc[0] = w[c / 2] >> (16 * (c & 1));
+                wc[0] = v.w[c / 2] >> (16 * (c & 1));
             }
             codes8<BITS>(wc, q);
 #pragma unroll
             for (int t = 0; t < 8; ++t) q[t] = __builtin_fmaf(q[t], s, b);
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
+                constexpr int XC = XDT == 2 ? 2 : 1;  // 16-byte pieces of 8 elements
+                u32x4_t xv[XC];
+#pragma unroll
+                for (int i = 0; i < XC; ++i)
+                    xv[i] = U > 1 ? v.x[(U > 1) * (XC * c + i)] : load_x(r, XC * c + i, v.kc);
                 float x[8];
-                const uint8_t* xs = xr[r] + (size_t)(kc + c * 8) * XB;
-                if constexpr (XDT == 2) {
-                    const f32x4_t v0 = *(const f32x4_t*)xs, v1 = *(const f32x4_t*)(xs + 16);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        x[e] = v0[e];
-                        x[4 + e] = v1[e];
-                    }
-                } else {
-                    const u32x4_t v = *(const u32x4_t*)xs;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        x[2 * e] = elem_to_f32<XDT == 1>(v[e] & 0xffffu);
-                        x[2 * e + 1] = elem_to_f32<XDT == 1>(v[e] >> 16);
+                for (int t = 0; t < 8; ++t) {
+                    if constexpr (XDT == 2) {
+                        x[t] = __uint_as_float(xv[t / 4][t & 3]);
+                    } else {
+                        const uint32_t e = xv[0][t / 2];
+                        x[t] = elem_to_f32<XDT == 1>(t & 1 ? e >> 16 : e & 0xffffu);
                     }
                 }
-                if (!in)  // lanes past K add nothing, whatever their row holds
+                if (!v.in)  // lanes past K add nothing, whatever their row holds
 #pragma unroll
                     for (int t = 0; t < 8; ++t) x[t] = 0.0f;
 #pragma unroll
@@ -660,7 +694,17 @@ __device__ __forceinline__ void qmm_f32(const QmmGenericParams& p) {
                                                                          acc[r][t & 3], 0, 0, 0);
             }
         }
-    }
+    };
+    int st = wave;
+    if constexpr (U > 1)
+        for (; st + (U - 1) * kF32Waves < steps; st += U * kF32Waves) {
+            Step v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = load(st + u * kF32Waves);
+#pragma unroll
+            for (int u = 0; u < U; ++u) add(v[u]);
+        }
+    for (; st < steps; st += kF32Waves) add(load(st));
 #pragma unroll
     for (int r = 0; r < RT; ++r)
         part[(wave * RT + r) * 64 + lane] = (acc[r][0] + acc[r][1]) + (acc[r][2] + acc[r][3]);

@@ -1460,6 +1460,32 @@ static dfq_status gemm_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const
  * then still has a step of 128 k. */
 static constexpr int kF32LongK = 2048;
 
+/* Row tiles of 16 (as a power of two) a workgroup of the fp32 kernel takes: as few as leave at
+ * most one workgroup a CU, else as many as the rows fill (up to 4).  Few columns are bound by a
+ * workgroup's chain of loads, which its row tiles lengthen.  Measured (us, 1 / 2 / 4 tiles), fp32
+ * x, bf16 scales, 4-bit: 64 x 16, K 4096 12.1 / 19.7 / 38.0; 64 x 1024, K 4096 (one tile 256
+ * workgroups) 17.7 / 21.5 / 39.5; 256 x 512 (two tiles 256) 36.1 / 29.1 / 43.1; 1024 x 512 118 /
+ * 100 / 108, 256 x 8192 450 / 367 / 372 (bf16 x, 8-bit 241 / 244 / 224). */
+static int f32_row_tiles(int M, int N, int num_cus) {
+    const int most = M <= 16 ? 0 : M <= 32 ? 1 : 2;
+    for (int r = 0; r < most; ++r)
+        if ((int64_t)((N + 15) / 16) * ((M + (16 << r) - 1) / (16 << r)) <= num_cus) return r;
+    return most;
+}
+
+/* Few outputs (four a CU, eight with fp32 scales) at K below 2048 in whole rounds of the
+ * per-element kernel's loads: that kernel, whose lanes take whole words over all CUs, where the
+ * fp32 kernel's take 8 k of their column in a few.  Measured (us, fp32 kernel / per element): fp32
+ * x over bf16 scales, 1 x 16, K 1024 5.1 / 4.6, 16 x 64 6.4 / 4.7; all fp32, 16 x 16, K 512 4.5 /
+ * 3.8, K 1536 8.3 / 6.0; fp16 x over fp32 scales, 8 x 256, K 1024 5.9 / 5.3; 2-bit bf16, 1 x 16, K
+ * 1024 5.4 / 4.5.  Elsewhere (K 544, 896, 1152; 16-bit operands at K 512, 768, 1280) the fp32
+ * kernel takes 0.7 to 1.1 of it. */
+static bool f32_per_element(int M, int N, int K, dfq_dtype xdt, dfq_dtype sdt, int num_cus) {
+    const bool any_f32 = xdt == DFQ_F32 || sdt == DFQ_F32;
+    return K < kF32LongK && (any_f32 ? K >= 512 && K % 256 == 0 : K >= 1024 && K % 512 == 0) &&
+           (int64_t)M * N <= (sdt == DFQ_F32 ? 8 : 4) * (int64_t)num_cus;
+}
+
 dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                             const void* biases, const void* lbias, void* y, int M, int N, int K,
                             int bits, int gs, dfq_dtype xdt, dfq_dtype sdt, dfq_dtype ydt,
@@ -1506,11 +1532,11 @@ dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, cons
     p.ydt = ydt;
     void* args[] = {&p};
     /* fp32 arithmetic on the matrix cores where a lane's codes and x are whole aligned loads
-     * in one group; otherwise one wave per output element */
+     * in one group (and the outputs are not too few); otherwise one wave per output element */
     const size_t sal = sdt == DFQ_F32 ? 4 : 2;
     if (K % 32 == 0 && gs % 32 == 0 && aligned(x, 16) && aligned(w, 16) && aligned(scales, sal) &&
-        aligned(biases, sal)) {
-        const int r = M <= 16 ? 0 : M <= 32 ? 1 : 2, k = K >= kF32LongK ? 1 : 0;
+        aligned(biases, sal) && !f32_per_element(M, N, K, xdt, sdt, ctx->num_cus)) {
+        const int r = f32_row_tiles(M, N, ctx->num_cus), k = K >= kF32LongK ? 1 : 0;
         hipError_t e = hipModuleLaunchKernel(
             ctx->f32[bits == 2 ? 0 : bits == 4 ? 1 : 2][k][(int)xdt][r], (unsigned)((N + 15) / 16),
             (unsigned)((M + (16 << r) - 1) / (16 << r)), 1, 1024, 1, 1, 0, (hipStream_t)stream,

@@ -8,8 +8,9 @@ from oracle.qmm_oracle import pack
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K, bits, gs, x dtype, scale dtype): one, two and four row tiles and their remainders,
-# ragged N, K below, at and past a whole round of 16 waves for either step, odd 32s of K
+# (M, N, K, bits, gs, x dtype, scale dtype): one row tile and its remainders, ragged N, K below, at
+# and past a whole round of 16 waves for either step, odd 32s of K; then grids of more than 256
+# workgroups, which take two and four row tiles, and outputs few enough for the per-element kernel
 CASES = [
     (1, 1, 32, 4, 32, "f32", "bf16"), (16, 17, 512, 4, 64, "f32", "bf16"),
     (17, 40, 544, 2, 32, "f32", "f16"), (32, 16, 2048, 8, 128, "bf16", "f16"),
@@ -17,6 +18,11 @@ CASES = [
     (65, 33, 1984, 8, 64, "f32", "f32"), (6, 4096, 4096, 4, 64, "f32", "bf16"),
     (5, 70, 6144, 8, 512, "f32", "bf16"), (3, 50, 96, 8, 96, "f32", "f16"),
     (130, 20, 4096, 4, 128, "f16", "f32"), (7, 90, 640, 2, 64, "bf16", "bf16"),
+    (5, 40, 1056, 4, 32, "f32", "bf16"),
+    (32, 2070, 544, 4, 32, "f32", "bf16"), (31, 2080, 2080, 8, 32, "bf16", "f16"),
+    (65, 1400, 160, 2, 32, "f32", "f16"), (129, 1391, 2080, 4, 32, "f16", "bf16"),
+    (3, 33, 1024, 2, 64, "bf16", "bf16"), (4, 60, 768, 8, 64, "f32", "f16"),
+    (8, 256, 1536, 4, 32, "f16", "f32"),
 ]
 
 
@@ -67,3 +73,19 @@ def test_padding_lanes_add_nothing(ctx):
     y = ctx.fallback(x, w, s, b, 4, 32)
     assert torch.equal(y[:-1, :-1], want[:-1, :-1])
     assert torch.isinf(y[-1]).all() and torch.isinf(y[:, -1]).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 1400, 544), (32, 2080, 2080), (200, 16, 4128)])
+def test_rows_do_not_depend_on_how_many_there_are(ctx, M, N, K):
+    """One, two and four row tiles a workgroup add the same products in the same order."""
+    import torch
+    rng = np.random.default_rng(M)
+    w = torch.from_numpy(pack(rng.integers(0, 16, size=(N, K), dtype=np.uint8), 4)
+                         .view(np.int32)).cuda()
+    x = torch.from_numpy(rng.normal(size=(M, K)).astype(np.float32)).cuda()
+    s = torch.full((N, K // 32), 0.5, dtype=torch.bfloat16, device="cuda")
+    b = torch.full_like(s, -3.75)
+    announce(f"stock fp32 rows M={M} N={N} K={K}")
+    y = ctx.fallback(x, w, s, b, 4, 32)
+    few = ctx.fallback(x[:9].contiguous(), w, s, b, 4, 32)
+    assert torch.equal(y[:9], few)
