@@ -1473,6 +1473,21 @@ static int f32_row_tiles(int M, int N, int num_cus) {
     return most;
 }
 
+/* Calls of one 16-bit dtype that go to the fp32 kernel where the GEMV does not take them: up to
+ * two row tiles over a long K, at most one workgroup a CU (two at up to 16 rows where the
+ * product's steps cost more: 8-bit codes, groups of 32).  The product is bound there by the chain
+ * of its steps over K in few workgroups, and fell behind the GEMV's launches it had replaced, or
+ * behind one wave an output.  Measured (us, GEMV / product / fp32 kernel): 8-bit fp16, groups
+ * of 128, 9 x 2048, K 17408 81 / 104 / 36, K 8192 44 / 48 / 19, K 5120 32 / 30 / -; groups of 64,
+ * 9 x 5120, K 17408 85 / 90 / 68; 4-bit bf16, groups of 64, 9 x 5120, K 17408 (more than one
+ * workgroup a CU) 72 / 61 / 63; past the GEMV's K, 4 x 40, K 24576 62 (one wave an output) / 67 /
+ * 44. */
+static bool f32_long_k(int M, int N, int K, int bits, int gs, int num_cus) {
+    const int64_t wgs = (int64_t)((N + 15) / 16) * ((M + 15) / 16);
+    return K >= 8192 && M <= 32 &&
+           wgs <= (M <= 16 && (bits == 8 || gs == 32) ? 2 : 1) * (int64_t)num_cus;
+}
+
 /* Few outputs (four a CU, eight with fp32 scales) at K below 2048 in whole rounds of the
  * per-element kernel's loads: that kernel, whose lanes take whole words over all CUs, where the
  * fp32 kernel's take 8 k of their column in a few.  Measured (us, fp32 kernel / per element): fp32
@@ -1510,7 +1525,7 @@ dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, cons
         if (M <= kQmvMaxRows)
             s = qmv_any(ctx, x, w, scales, biases, lbias, y, M, N, K, bits, gs, xdt,
                         (hipStream_t)stream);
-        if (s == DFQ_ERR_UNSUPPORTED)
+        if (s == DFQ_ERR_UNSUPPORTED && !f32_long_k(M, N, K, bits, gs, ctx->num_cus))
             s = gemm_any(ctx, x, w, scales, biases, lbias, y, M, N, K, bits, gs, xdt,
                          (hipStream_t)stream);
         if (s != DFQ_ERR_UNSUPPORTED) return s;

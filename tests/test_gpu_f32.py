@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 # (M, N, K, bits, gs, x dtype, scale dtype): one row tile and its remainders, ragged N, K below, at
 # and past a whole round of 16 waves for either step, odd 32s of K; then grids of more than 256
-# workgroups, which take two and four row tiles, and outputs few enough for the per-element kernel
+# workgroups, which take two and four row tiles, and outputs few enough for the per-element kernel;
+# last, one dtype over a long K, which the product and the GEMV leave to this kernel
 CASES = [
     (1, 1, 32, 4, 32, "f32", "bf16"), (16, 17, 512, 4, 64, "f32", "bf16"),
     (17, 40, 544, 2, 32, "f32", "f16"), (32, 16, 2048, 8, 128, "bf16", "f16"),
@@ -23,6 +24,9 @@ CASES = [
     (65, 1400, 160, 2, 32, "f32", "f16"), (129, 1391, 2080, 4, 32, "f16", "bf16"),
     (3, 33, 1024, 2, 64, "bf16", "bf16"), (4, 60, 768, 8, 64, "f32", "f16"),
     (8, 256, 1536, 4, 32, "f16", "f32"),
+    (9, 40, 8192, 8, 128, "bf16", "bf16"), (16, 33, 8224, 4, 32, "f16", "f16"),
+    (32, 17, 17408, 4, 64, "bf16", "bf16"), (1, 40, 40960, 4, 64, "bf16", "bf16"),
+    (4, 21, 24576, 8, 128, "f16", "f16"),
 ]
 
 

@@ -59,10 +59,10 @@ def test_matches_oracle(ctx, oracle, M, N, bits, gs, dt):
 
 
 def test_rows_past_the_gemvs_limit_in_k_and_misaligned_scales(ctx, oracle):
-    """K too long for the GEMV's x in LDS takes the product at any M, and scales that are not
-    aligned for a line's vector load are read one by one."""
+    """A long K, and scales that are not aligned for a line's vector load, which are read one by
+    one: the same bits."""
     import torch
-    c = make_case(3, 40, 32768, bits=4, gs=64, seed=5)
+    c = make_case(40, 40, 32768, bits=4, gs=64, seed=5)
     x, w, s, b, _ = upload(c)
     assert ctx.stock_gemv_launches(3, 40, 32768, 4, 64) == 0
     announce("stock gemm long K")
