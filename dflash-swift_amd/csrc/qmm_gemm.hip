@@ -514,22 +514,24 @@ __device__ __forceinline__ void qmm_gemm(const QmmGemmParams& p) {
         qmm_gemm<BITS, GS, F16, RT, CT, MW, NW, KW>(p);                                      \
     }
 /* rows x columns of a workgroup's tile, and slices of K (kGemmTiles in qmm_runtime.cpp) */
-#define DFQ_GEMM_FORMAT(BITS, GS, F16, NAME)                         \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 128x128, 4, 1, 1, 4, 1)     \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 96x128, 3, 1, 1, 4, 1)      \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128, 2, 1, 1, 4, 1)      \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128_k2, 2, 1, 1, 4, 2)   \
-    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x128_k2, 1, 1, 1, 4, 2)   \
+#define DFQ_GEMM_FORMAT(BITS, GS, F16, NAME)                       \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 96x128, 3, 1, 1, 4, 1)    \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128, 2, 1, 1, 4, 1)    \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 64x128_k2, 2, 1, 1, 4, 2) \
+    DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x128_k2, 1, 1, 1, 4, 2) \
     DFQ_GEMM_KERNEL(BITS, GS, F16, NAME, 32x64_k4, 1, 1, 1, 2, 4)
+#define DFQ_GEMM_FORMAT64(BITS, F16, NAME)                        \
+    DFQ_GEMM_KERNEL(BITS, 64, F16, NAME, 128x128, 4, 1, 1, 4, 1) \
+    DFQ_GEMM_FORMAT(BITS, 64, F16, NAME)
 
 DFQ_GEMM_FORMAT(4, 32, false, bf16)
-DFQ_GEMM_FORMAT(4, 64, false, bf16)
+DFQ_GEMM_FORMAT64(4, false, bf16)
 DFQ_GEMM_FORMAT(8, 32, false, bf16)
-DFQ_GEMM_FORMAT(8, 64, false, bf16)
+DFQ_GEMM_FORMAT64(8, false, bf16)
 DFQ_GEMM_FORMAT(4, 32, true, f16)
-DFQ_GEMM_FORMAT(4, 64, true, f16)
+DFQ_GEMM_FORMAT64(4, true, f16)
 DFQ_GEMM_FORMAT(8, 32, true, f16)
-DFQ_GEMM_FORMAT(8, 64, true, f16)
+DFQ_GEMM_FORMAT64(8, true, f16)
 
 /* ---------------------------------------------------------------------------------- */
 /* The stock path in fp32: promoted dtypes, fp32 arrays, 2-bit codes, other groups      */

@@ -111,17 +111,18 @@ struct GemmTile {
     const char* name;
     int rows, cols, threads;
     int per_cu;   /* workgroups a CU holds (LDS) */
-    float alone;  /* us per 64 k of a workgroup that has its CU to itself */
     float full;   /* us per 64 k and round of per_cu workgroups */
+    float alone;  /* us per 64 k of the one workgroup of a last round (per_cu 2 only) */
 };
 constexpr int kGemmTileCount = 6;
+constexpr int kGemmFirst32 = 1;  /* the first tile built for groups of 32 */
 static const GemmTile kGemmTiles[kGemmTileCount] = {
-    {"128x128", 128, 128, 256, 2, 0.83f, 1.52f},
-    {"96x128", 96, 128, 256, 2, 0.69f, 1.22f},
-    {"64x128", 64, 128, 256, 2, 0.59f, 0.90f},
-    {"64x128_k2", 64, 128, 512, 1, 0.50f, 0.55f},
-    {"32x128_k2", 32, 128, 512, 1, 0.396f, 0.385f},
-    {"32x64_k4", 32, 64, 512, 1, 0.249f, 0.24f},
+    {"128x128", 128, 128, 256, 2, 1.52f, 0.83f},  /* not built for groups of 32 (see gemm_tile) */
+    {"96x128", 96, 128, 256, 2, 1.22f, 0.69f},
+    {"64x128", 64, 128, 256, 2, 0.90f, 0.59f},
+    {"64x128_k2", 64, 128, 512, 1, 0.55f, 0.0f},
+    {"32x128_k2", 32, 128, 512, 1, 0.385f, 0.0f},
+    {"32x64_k4", 32, 64, 512, 1, 0.24f, 0.0f},
 };
 
 struct dfq_ctx {
@@ -589,7 +590,7 @@ static dfq_status load_gemm(dfq_ctx* ctx) {
     for (int b = 0; b < 2; ++b)
         for (int g = 0; g < 2; ++g)
             for (int d = 0; d < 2; ++d)
-                for (int t = 0; t < kGemmTileCount; ++t) {
+                for (int t = g ? 0 : kGemmFirst32; t < kGemmTileCount; ++t) {
                     char name[64];
                     snprintf(name, sizeof name, "dfq_gemm_b%d_g%d_%s_%s", b ? 8 : 4, g ? 64 : 32,
                              d ? "f16" : "bf16", kGemmTiles[t].name);
@@ -1397,22 +1398,27 @@ static dfq_status qmv_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const 
     return DFQ_OK;
 }
 
-/* The tile that finishes first by its measured step times: a CU works through its share of the
- * tiles in rounds of per_cu workgroups, and an odd last one has the CU to itself.  Measured on
- * MI355X (us, each tile in the table's order; the model picks the best or one within 6 % of it):
- * 2048 x 17408, K 5120, 4-bit bf16: 513 569 644 735 1042 1220; 512 x 5120, K 5120: 68 61 70 88
- * 102 98; 200 x 17408, K 5120: 107 89 112 118 114 131; 333 x 5120, K 17408, 8-bit fp16: 245 212
- * 189 187 248 297; 64 x 5120, K 5120: 66 55 49 40 31 20; 16 x 17408, K 5120: 69 57 49 41 32 38. */
-static int gemm_tile(int M, int N, int num_cus) {
-    int best = 0;
+/* The tile that finishes first by step times measured in 4-bit bf16, groups of 64, for all
+ * formats: a CU works through its share of the tiles in rounds of per_cu workgroups, and an odd
+ * last one has the CU to itself.  Measured on MI355X (us, each tile in the table's order): groups
+ * of 64, 4-bit bf16, K 5120, 2048 x 17408 530 596 682 743 1061 1232; 512 x 5120 69 62 69 79 89 87;
+ * 200 x 17408 106 92 118 121 128 140; 100 x 5120 69 60 51 40 31 35; 12 x 5120 68 59 51 40 30 18.
+ * Over 12 to 2048 rows, 1024 to 17408 columns, K 5120, the pick is the best or within 2 % of it
+ * there, 5 % in 8 bits, 11 % in groups of 128.  128 x 128 in groups of 32 spilled 13 to 28
+ * registers in the step and lost to 96 x 128 wherever it was picked but once (2048 x 17408 867
+ * against 718, 512 x 17408 288 against 224, 100 x 17408 135 against 90 in 64 x 128; 333 x 17408
+ * 165 against 177): without it the pick is within 9 %. */
+static int gemm_tile(int M, int N, int gs, int num_cus) {
+    const int first = gs == 32 ? kGemmFirst32 : 0;
+    int best = first;
     double least = 0;
-    for (int i = 0; i < kGemmTileCount; ++i) {
+    for (int i = first; i < kGemmTileCount; ++i) {
         const GemmTile& t = kGemmTiles[i];
         const int64_t tiles = (int64_t)((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
         const int64_t share = (tiles + num_cus - 1) / num_cus;
         const double us = (double)(share / t.per_cu) * t.full +
                           (share % t.per_cu ? (double)t.alone : 0.0);
-        if (i == 0 || us < least) {
+        if (i == first || us < least) {
             least = us;
             best = i;
         }
@@ -1428,7 +1434,7 @@ static dfq_status gemm_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const
                            int bits, int gs, dfq_dtype dt, hipStream_t stream) {
     if (!stock_format(bits, gs, dt, x, w, scales, biases, y) || K > (1 << 22))
         return DFQ_ERR_UNSUPPORTED;
-    const int ti = gemm_tile(M, N, ctx->num_cus);
+    const int ti = gemm_tile(M, N, gs, ctx->num_cus);
     const GemmTile& t = kGemmTiles[ti];
     const int gk = gs == 32 ? 32 : 64;          // the kernel's group
     const int lg = 1024 / bits / gk;            // its groups in a 128-byte line of codes
