@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 FORMATS = [(bits, gs, dt) for bits in (4, 8) for gs in (32, 64, 128) for dt in (BF16, F16)]
 # (rows, columns) that take each tile of the dispatch on 256 CUs, with ragged edges: 32 x 64 in
-# four K slices (twice), 32 x 128 and 64 x 128 in two, 64 x 128, 96 x 128, 128 x 128
+# four K slices (twice), 32 x 128 and 64 x 128 in two, 64 x 128, 96 x 128, 128 x 128 (96 x 128 in
+# groups of 32)
 TILES = [(9, 37), (33, 130), (32, 17000), (64, 16397), (385, 9001), (65, 16397), (400, 14001)]
 
 
@@ -41,7 +42,7 @@ def test_one_hot_rows_are_exact(ctx, bits, gs, dt):
 @pytest.mark.parametrize("M,N", TILES)
 def test_matches_oracle(ctx, oracle, M, N, bits, gs, dt):
     """|y - y64| <= u_out |y64| + (K + 8) 2^-24 S, S = sum |x| (|s| (MAGIC + q_max) + |b|): one
-    output rounding and at most K + 8 roundings of sums no larger than S (MAGIC 128 at bf16
+    output rounding and at most K + 8 roundings of sums no larger than S (MAGIC 16 at bf16
     4-bit, 0 otherwise), + one unit of the smallest fp16."""
     K = {32: 352, 64: 704, 128: 640}[gs] if N < 6000 else 3 * gs
     c = make_case(M, N, K, bits=bits, gs=gs, xdt=dt, seed=M + N + bits, lbias=(M % 2 == 1))
@@ -49,13 +50,77 @@ def test_matches_oracle(ctx, oracle, M, N, bits, gs, dt):
     announce(f"stock gemm M={M} N={N} K={K} bits={bits} gs={gs} dt={dt}")
     y = download(ctx.fallback(x, w, s, b, bits, gs, lbias=lb))
     ref = oracle.qmm_f64(c)
-    top = (1 << bits) - 1 + (128 if bits == 4 and dt == BF16 else 0)
+    top = (1 << bits) - 1 + (16 if bits == 4 and dt == BF16 else 0)
     wmax = np.repeat(np.abs(download(s)) * top + np.abs(download(b)), gs, axis=1)
     S = np.abs(download(x)) @ wmax.T + (0 if lb is None else np.abs(download(lb)))
     u = 2.0 ** -8 if dt == BF16 else 2.0 ** -11  # half a unit of 8 and 11 significant bits
     bound = u * np.abs(ref) + (K + 8) * 2.0 ** -24 * S + 2.0 ** -24
     bad = np.argwhere(~(np.abs(y - ref) <= bound))
     assert bad.size == 0, (len(bad), bad[0], y[tuple(bad[0])], ref[tuple(bad[0])])
+
+
+def dequantised(w, s, b, bits, gs):
+    """Rows of the weight in float64, on the GPU."""
+    import torch
+    per = 32 // bits
+    q = torch.stack([(w >> (bits * t)) & ((1 << bits) - 1) for t in range(per)], 2)
+    q = q.reshape(w.shape[0], -1, gs).double()
+    return (q * s.double()[:, :, None] + b.double()[:, :, None]).reshape(w.shape[0], -1)
+
+
+@pytest.mark.parametrize("bits,gs,dt", FORMATS)
+@pytest.mark.parametrize("M,N", TILES)
+@pytest.mark.parametrize("ragged", [False, True])
+def test_every_tile_over_many_lines_and_slices(ctx, M, N, bits, gs, dt, ragged):
+    """38 to 40 steps of 64 k: every slice of K has work, code and scale buffers and X sets are
+    used again in each, with whole lines of scales (vector loads, groups of 32 and 64) and with a
+    last line, set and step that are not whole.  Against float64 at the first and last columns and
+    a sample, with the bound of test_matches_oracle; and a row's bits depend on that row alone,
+    among calls of as many rows."""
+    import torch
+    K = {32: 2464, 64: 2496, 128: 2432}[gs] if ragged else 2560
+    tdt = torch.bfloat16 if dt == BF16 else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(M + N + bits + gs + dt)
+    w = torch.randint(-2**31, 2**31, (N, K * bits // 32), dtype=torch.int64, device="cuda",
+                      generator=g).to(torch.int32)
+    r = lambda *size: torch.randn(*size, device="cuda", generator=g)
+    s, b = (r(N, K // gs) * 0.02).to(tdt), (r(N, K // gs) * 0.1).to(tdt)
+    x, lb = r(M, K).to(tdt), r(N).to(tdt)
+    announce(f"stock gemm tiles M={M} N={N} K={K} bits={bits} gs={gs} dt={dt}")
+    y = ctx.fallback(x, w, s, b, bits, gs, lbias=lb).double()
+    c = torch.cat([torch.arange(min(N, 40)), torch.randint(0, N, (200,)),
+                   torch.arange(max(0, N - 140), N)]).cuda()
+    ref = x.double() @ dequantised(w[c], s[c], b[c], bits, gs).t().contiguous() + lb[c].double()
+    top = (1 << bits) - 1 + (16 if bits == 4 and dt == BF16 else 0)
+    wmax = (s[c].double().abs() * top + b[c].double().abs()).repeat_interleave(gs, 1)
+    S = x.double().abs() @ wmax.t().contiguous() + lb[c].double().abs()
+    u = 2.0 ** -8 if dt == BF16 else 2.0 ** -11
+    bound = u * ref.abs() + (K + 8) * 2.0 ** -24 * S + 2.0 ** -24
+    bad = ((y[:, c] - ref).abs() > bound).nonzero().cpu()
+    assert len(bad) == 0 and bool(torch.isfinite(y).all()), (len(bad), bad[:3])
+    x[1:] = r(M - 1, K).to(tdt)
+    assert torch.equal(ctx.fallback(x, w, s, b, bits, gs, lbias=lb)[0].double(), y[0])
+
+
+@pytest.mark.parametrize("bits,gs,dt", FORMATS)
+@pytest.mark.parametrize("M,N", TILES)
+def test_one_hot_rows_are_exact_in_every_tile(ctx, M, N, bits, gs, dt):
+    """M positions of K over all slices, lines and steps, 53 weight rows repeated over N."""
+    import torch
+    K = {32: 2464, 64: 2496, 128: 2432}[gs]
+    w, sb, bb, deq = exact_case(53, K, bits, gs, dt, seed=bits * 10 + gs + dt)
+    n = np.arange(N) % 53
+    k = np.concatenate([[0, K - 1], np.linspace(1, K - 2, M - 2).astype(int)])
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).cuda()
+    tdt = torch.bfloat16 if dt == BF16 else torch.float16
+    wd = torch.from_numpy(w.view(np.int32)).cuda()[torch.from_numpy(n).cuda()].contiguous()
+    sd, bd = (dev(a)[torch.from_numpy(n).cuda()].contiguous().view(tdt) for a in (sb, bb))
+    x = torch.zeros(M, K, dtype=tdt, device="cuda")
+    x[torch.arange(M), torch.from_numpy(k)] = 1.0
+    announce(f"stock gemm one-hot tiles M={M} N={N} bits={bits} gs={gs} dt={dt}")
+    y = ctx.fallback(x, wd, sd, bd, bits, gs)
+    want = dev(to_bits(deq[:, k].T, dt))[:, torch.from_numpy(n).cuda()]
+    assert torch.equal(y.view(torch.int16), want)
 
 
 def test_rows_past_the_gemvs_limit_in_k_and_misaligned_scales(ctx, oracle):

@@ -320,13 +320,13 @@ def test_sixteen_rows_take_one_launch(ctx):
     assert p["ch"] > 1 and p["T"] == 1088
 
 
-def test_kernel_output_is_not_the_generic_path(ctx):
+def test_kernel_output_is_not_the_stock_path(ctx):
     """Negative control (SmallMQuantizedMatmulTests.swift:94-102): the fast kernel's
-    accumulation order differs from the generic path's, so at least one output moves."""
+    accumulation order differs from the stock path's, so at least one output moves."""
     import torch
     c = config_case("c2_gateup_k5120_n17408", 8)
     x, w, s, b, _ = upload(c)
-    announce("negative control c2 M=8 fast vs generic")
+    announce("negative control c2 M=8 fast vs stock")
     fast = ctx.qmm(x, w, s, b, 4, 64)
     slow = ctx.fallback(x, w, s, b, 4, 64)
     assert slow.dtype == fast.dtype
@@ -335,24 +335,61 @@ def test_kernel_output_is_not_the_generic_path(ctx):
     assert rel <= TOL and ok
 
 
-def test_generic_path_matches_oracle(ctx, oracle):
+def test_stock_path_matches_oracle(ctx, oracle):
     for (M, N, K, bits, gs, dt) in [(3, 50, 256, 4, 64, BF16), (2, 40, 256, 8, 32, F16),
                                     (4, 33, 512, 2, 64, BF16), (5, 64, 384, 4, 128, BF16)]:
         c = make_case(M, N, K, bits=bits, gs=gs, xdt=dt, seed=K + N, lbias=True)
         x, w, s, b, lb = upload(c)
-        announce(f"generic M={M} N={N} K={K} bits={bits} gs={gs}")
+        announce(f"stock M={M} N={N} K={K} bits={bits} gs={gs}")
         y = download(ctx.fallback(x, w, s, b, bits, gs, lbias=lb))
         rel, ok = tolerance_check(y, oracle.qmm_f64(c))
         assert rel <= TOL and ok, (M, N, K, bits, gs, rel)
 
 
-def test_generic_path_promotes_mixed_dtypes(ctx, oracle):
-    """fp16 x against bf16 scales: MLX promotes to fp32, and so does the generic path."""
+def test_stock_path_promotes_mixed_dtypes(ctx, oracle):
+    """fp16 x against bf16 scales: MLX promotes to fp32, and so does the stock path."""
     import torch
     c = make_case(4, 64, 256, bits=4, gs=64, xdt=F16, sdt=BF16, seed=9)
     x, w, s, b, _ = upload(c)
-    announce("generic mixed dtype")
+    announce("stock mixed dtype")
     y = ctx.fallback(x, w, s, b, 4, 64)
     assert y.dtype == torch.float32
     rel, ok = tolerance_check(download(y), oracle.qmm_f64(c))
     assert rel <= 1e-5 and ok
+
+
+# (M, N, K, bits, gs, x dtype, scale dtype, element x is off its alignment by, word w is off by):
+# groups and lengths that are no multiples of 32, arrays that are not 16-byte aligned, rows on both
+# sides of 8, one dtype and two
+PER_ELEMENT = [
+    (3, 50, 256, 4, 16, BF16, BF16, 0, 0), (17, 33, 200, 4, 40, F16, F16, 0, 0),
+    (9, 40, 272, 2, 16, BF16, F16, 0, 0), (5, 37, 256, 4, 64, BF16, BF16, 1, 0),
+    (12, 64, 512, 8, 32, F16, F16, 1, 0), (2, 20, 320, 4, 64, F16, BF16, 1, 0),
+    (10, 35, 384, 8, 128, BF16, BF16, 0, 1), (33, 70, 256, 2, 64, F16, F16, 0, 3),
+    (4, 21, 36, 8, 4, BF16, BF16, 0, 0),
+]
+
+
+@pytest.mark.parametrize("case", PER_ELEMENT)
+def test_per_element_kernel_matches_oracle(ctx, oracle, case):
+    """What neither the GEMV nor the products take, one wave an output: |y - y64| <= u_out |y64| +
+    (K + 24) 2^-24 S, S = sum |x| (|s| q_max + |b|) + |linear bias|."""
+    import torch
+    M, N, K, bits, gs, xdt, sdt, xoff, woff = case
+    c = make_case(M, N, K, bits=bits, gs=gs, xdt=xdt, sdt=sdt, seed=M + N, lbias=True)
+    x, w, s, b, lb = upload(c)
+
+    def moved(t, off):
+        buf = torch.empty(t.numel() + 16, dtype=t.dtype, device="cuda")
+        assert buf.data_ptr() % 16 == 0
+        return buf[off:off + t.numel()].view(t.shape).copy_(t)
+
+    x, w = moved(x, xoff), moved(w, woff)
+    announce(f"stock per element {case}")
+    y = ctx.fallback(x, w, s, b, bits, gs, lbias=lb)
+    assert y.dtype == (x.dtype if xdt == sdt else torch.float32)
+    ref = oracle.qmm_f64(c)
+    wmax = np.repeat(np.abs(download(s)) * ((1 << bits) - 1) + np.abs(download(b)), gs, axis=1)
+    S = np.abs(download(x)) @ wmax.T + np.abs(download(lb))
+    u = 0.0 if xdt != sdt else 2.0 ** -8 if xdt == BF16 else 2.0 ** -11
+    assert (np.abs(download(y) - ref) <= u * np.abs(ref) + (K + 24) * 2.0 ** -24 * S).all()

@@ -9,7 +9,7 @@ weight row read once a launch.  Pinned three ways:
   oracle's dequant bit for bit, at every k position of several lane chunks, in every format;
 * against the fp64 oracle at 1..8 rows (5..8 rows take two launches), ragged N, K whose last
   step covers part of the lanes, a linear bias, and the benchmark shapes at full size;
-* the path taken: the GEMV, not the per-element kernel, for these shapes.
+* the path taken: the GEMV, not another kernel, for these shapes.
 """
 import numpy as np
 import pytest
@@ -109,7 +109,7 @@ def test_stock_gemv_is_deterministic_and_row_independent(ctx):
     assert eq(y4[:3], y3) and eq(y7[:4], y4) and eq(y7[4:], y3)
 
 
-def test_mixed_dtypes_and_two_bit_codes_take_the_per_element_path(ctx):
+def test_two_bit_codes_and_other_groups_are_not_the_gemvs(ctx):
     assert ctx.stock_gemv_launches(4, 64, 256, 2, 64, BF16) == 0
     assert ctx.stock_gemv_launches(4, 64, 256, 4, 16, BF16) == 0
     assert ctx.stock_gemv_launches(4, 64, 200, 4, 40, BF16) == 0
