@@ -607,7 +607,7 @@ __device__ __forceinline__ void qmm_f32(const QmmGenericParams& p) {
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int a = 0; a < 4; ++a) acc[r][a] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    const int steps = (K + 4 * KL - 1) / (4 * KL);
+    const int steps = (K - 1) / (4 * KL) + 1;
     constexpr int XW = XDT == 2 ? KL / 4 : KL / 8;  // 16-byte loads of a lane's x of one row
     constexpr int WD = CB < 4 ? 1 : CB / 4;         // words of its codes
     struct Step {
@@ -622,9 +622,11 @@ __device__ __forceinline__ void qmm_f32(const QmmGenericParams& p) {
     };
     auto load = [&](int st) {
         Step v;
-        const int k = st * 4 * KL + j * KL;
-        const bool in = k < K;  // (K is a multiple of KL) lanes past K read its last codes
-        const int kc = in ? k : K - KL;
+        /* (unsigned: the last step of a K near 2^31 ends past it.  K is a multiple of KL) lanes
+         * past K read its last codes */
+        const uint32_t k = (uint32_t)st * (4 * KL) + (uint32_t)(j * KL);
+        const bool in = k < (uint32_t)K;
+        const int kc = in ? (int)k : K - KL;
         const uint8_t* ws = wr + (size_t)kc * BITS / 8;
         if constexpr (CB == 2) {
             v.w[0] = *(const uint16_t*)ws;
