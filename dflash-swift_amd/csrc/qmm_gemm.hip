@@ -43,12 +43,14 @@
  * The next step is staged after all but the last two row tiles' LDS reads, which its writes
  * would otherwise hold up (2048 x 17408, K 5120: 527 us after the first, 513).
  *
- * Measured on MI355X against the GEMV's launches it replaces (us): 512 x 5120, K 5120, 4-bit
- * bf16 1537 -> 58.6; 2048 x 17408, K 5120 12548 -> 517 (706 TFLOP/s); an MLP of 333 rows, 8-bit
- * fp16 6565 -> 432.  Bound by the issue of vector instructions next to the matrix pipe: a
- * wave's step of 128 x 32 has about 700 matrix cycles and 150 vector instructions, up to six of
- * which issue behind an MFMA of their own wave, but another wave's only one (measured: an FMA
- * every 32 cycles beside a wave of MFMAs), so two waves a SIMD hardly fill each other's gaps.
+ * Measured on MI355X against the GEMV's launches it replaces (us a pass): 512 x 5120, K 5120,
+ * 4-bit bf16 1537 -> 59.9; 2048 x 17408, K 5120 12548 -> 527 (693 TFLOP/s); an MLP of 333 rows,
+ * 8-bit fp16 6566 -> 423.  A wave's step of 128 x 32 has 704 matrix cycles, of which 512 are the
+ * product, 128 the x sums (31 of 32 columns of ones . x are the same) and 64 the X products, and
+ * about 150 vector instructions, up to six of which issue behind an MFMA of their own wave, but
+ * another wave's only one (measured: an FMA every 32 cycles beside a wave of MFMAs), so two waves a
+ * SIMD hardly fill each other's gaps.  Where a grid leaves one workgroup a CU (512 x 5120: 240)
+ * there is one wave a SIMD, and LDS reads, vector work and MFMAs add up.
  */
 #include "qmm_device.h"
 #include "qmm_params.h"
@@ -581,9 +583,10 @@ __device__ __forceinline__ float bits_to_f32(uint32_t v, int dt) {
  * With one row tile the loads of two of a wave's steps are issued together (more tiles would
  * spill): 16 x 16, K 17408, all fp32 58.7 -> 48.7 us.
  *
- * Measured on MI355X, fp32 x over bf16 scales, 6 x 4096, K 4096, 4-bit: 172.4 us by the
- * per-element kernel, 12.6 a pass here; both are 1.6e-7 from the 64-bit result.  Bound by latency: a wave
- * has two steps. */
+ * Measured on MI355X, fp32 x over bf16 scales, 6 x 4096, K 4096, 4-bit: 172 us a pass by the
+ * per-element kernel, 12.5 here, 10 to 11 of them the kernel; both are 1.6e-7 from the 64-bit
+ * result.  Bound by latency, a wave has two steps, and by the 16 rows of a tile that 6 fill (3.4 us
+ * of matrix time). */
 template <int BITS, int KL, int XDT, int RT>
 __device__ __forceinline__ void qmm_f32(const QmmGenericParams& p) {
     __shared__ f32x4_t part[kF32Waves * RT * 64];

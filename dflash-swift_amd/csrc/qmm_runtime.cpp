@@ -1368,7 +1368,7 @@ static bool qmv_layout(const dfq_ctx* ctx, int M, int N, int K, int bits, QmvPar
 /* The stock path as MLX takes it for few rows: its GEMV, one launch per 4 rows, for one dtype
  * of x, scales, biases and y (bf16 or fp16), 4- or 8-bit codes, group 32, 64 or 128, K a
  * multiple of one lane's chunk, and x of 4 rows in LDS; DFQ_ERR_UNSUPPORTED otherwise (the
- * per-element path then takes the call). */
+ * product or the fp32 kernel then takes the call). */
 static dfq_status qmv_any(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                           const void* biases, const void* lbias, void* y, int M, int N, int K,
                           int bits, int gs, dfq_dtype dt, hipStream_t stream) {
@@ -1515,9 +1515,9 @@ dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, cons
     if (!x || !w || !scales || !biases || !y)
         return fail(DFQ_ERR_INVALID_ARGUMENT, "null x, w, scales, biases or y");
     if (M < 1 || N < 1 || K < 1) return fail(DFQ_ERR_INVALID_ARGUMENT, "M, N, K must be >= 1");
-    if (M > 65535) return fail(DFQ_ERR_UNSUPPORTED, "generic path handles M <= 65535");
+    if (M > 65535) return fail(DFQ_ERR_UNSUPPORTED, "the stock path handles M <= 65535");
     if (bits != 2 && bits != 4 && bits != 8)
-        return fail(DFQ_ERR_UNSUPPORTED, "generic path handles bits 2, 4, 8 (got %d)", bits);
+        return fail(DFQ_ERR_UNSUPPORTED, "the stock path handles bits 2, 4, 8 (got %d)", bits);
     if (gs < 32 / bits || gs <= 0 || K % gs || (gs % (32 / bits)))
         return fail(DFQ_ERR_UNSUPPORTED, "group size %d must divide K=%d and hold whole words",
                     gs, K);

@@ -99,7 +99,7 @@ public:
         if (took) *took = 0;
         if (packedOnly()) return packedSlices(x, xdt, rows, y, ws, wsb, stream);
         if (!d_.biases)
-            return dfq::fail(DFQ_ERR_UNSUPPORTED, "the generic path needs affine biases");
+            return dfq::fail(DFQ_ERR_UNSUPPORTED, "the stock path needs affine biases");
         return dfq_qmm_fallback(ctx_, x, d_.weight, d_.scales, d_.biases, d_.bias, y, rows,
                                 d_.out_features, d_.in_features, d_.bits, d_.group_size, xdt,
                                 d_.dtype, outputDType(xdt), stream);

@@ -256,7 +256,7 @@ class Context:
         return dict(zip(keys, list(out)))
 
     def stock_gemv_launches(self, M, N, K, bits, gs, dt=BF16) -> int:
-        """GEMV launches the stock path makes for a shape (0: the per-element path)."""
+        """GEMV launches the stock path makes for a shape (0: another kernel)."""
         n = ctypes.c_int(-1)
         _check(self.lib.dfq_debug_stock_gemv_launches(self.handle, M, N, K, bits, gs, dt,
                                                       ctypes.byref(n)),

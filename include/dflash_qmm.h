@@ -172,11 +172,21 @@ dfq_status dfq_interleave_gate_up(dfq_ctx* ctx, const void* gate, const void* up
  * at SmallMQuantizedMatmul.swift:265), which runs a GEMV for few rows.  Where x, scales and y
  * share bf16 or fp16, bits are 4 or 8 and the group 32, 64 or 128, up to 8 rows run as that
  * GEMV where 4 rows of x fit in LDS, one launch per 4 rows (each weight row read once a launch),
- * and more rows as one matrix product on the matrix cores (its sums in another order).  Every
- * other call has fp32 weights, products and sums: on the fp32 matrix instruction where K and the
- * group are multiples of 32 and x and w are 16-byte aligned, else one wave per output element,
- * re-reading W for every row.  No workspace; asynchronous on
- * `stream`. */
+ * and more rows as one matrix product on the matrix cores (its sums in another order); up to 32
+ * rows of few columns over a K from 8192 that the GEMV does not take run as the calls below.
+ * Every other call has fp32 weights, products and sums: on the fp32 matrix instruction where K and
+ * the group are multiples of 32 and x and w are 16-byte aligned, else (and for few outputs at some
+ * K below 2048) one wave per output element, re-reading W for every row.  M is at most 65535.
+ *
+ * The same call gives the same bits every time, and a row's result depends on its own x alone.
+ * It also depends on M, in the last bits, where M changes the kernel (GEMV, product, fp32) or the
+ * product's tile, whose slices of K are summed apart: a prompt in chunks is not bit for bit the
+ * whole one.  Among rows that the GEMV takes, and among those of the fp32 kernel, it does not.
+ *
+ * Infinities and NaN: the GEMV and the product sum s P and b X (x against the codes, and x's
+ * sums against the bias) apart, so an infinite x gives NaN where the two are infinities of
+ * opposite sign, also where the weight itself is of one sign; never an infinity of the wrong
+ * sign.  No workspace; asynchronous on `stream`. */
 dfq_status dfq_qmm_fallback(dfq_ctx* ctx, const void* x, const uint32_t* w, const void* scales,
                             const void* biases, const void* linear_bias, void* y, int M, int N,
                             int K, int bits, int group_size, dfq_dtype x_dtype,
@@ -306,7 +316,7 @@ typedef struct dfq_linear_desc {
     dfq_dtype dtype;          /* dtype of scales / biases / bias                     */
 } dfq_linear_desc;
 
-/* A stock QuantizedLinear: every call goes to the generic path.  ctx may be NULL for a
+/* A stock QuantizedLinear: every call goes to the stock path.  ctx may be NULL for a
  * layer that is only inspected or swapped (its forward then returns DFQ_ERR_STATE). */
 dfq_status dfq_linear_create(dfq_ctx* ctx, const dfq_linear_desc* desc, dfq_linear** out);
 /* SmallMQuantizedLinear(other): wraps `other`, sharing its arrays (:243-252). */

@@ -2,7 +2,7 @@
 
 CPU: both oracle restatements reproduce every stored dequant bit for bit and every stored
 fp64 result, and the known-answer unpack words decode as stored.  GPU: the fast kernel and
-the generic path meet the 1e-2 bar on every fixture.
+the stock path meet the 1e-2 bar on every fixture.
 """
 import os
 

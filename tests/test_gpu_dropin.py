@@ -1,7 +1,7 @@
 """The drop-in layer on the GPU, mirroring the reference's kernel tests.
 
 Reference: Tests/DFlashKitTests/SmallMQuantizedMatmulTests.swift.  `stock` is a plain
-QuantizedLinear (the generic path), `fast` is SmallMQuantizedLinear(stock) sharing its
+QuantizedLinear (the stock path), `fast` is SmallMQuantizedLinear(stock) sharing its
 arrays.  The reference builds its layer with MLX's quantiser from normal(scale 0.05) weights
 (:47-55); MLX is not available here, so codes, scales and biases are drawn directly with the
 same layer shape (out 4096, in 1024, group 64).
