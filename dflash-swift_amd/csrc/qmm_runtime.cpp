@@ -1484,13 +1484,13 @@ static int f32_row_tiles(int M, int N, int num_cus) {
  * product's steps cost more: 8-bit codes, groups of 32).  The product is bound there by the chain
  * of its steps over K in few workgroups, and fell behind the GEMV's launches it had replaced, or
  * behind one wave an output.  Measured (us, GEMV / product / fp32 kernel): 8-bit fp16, groups
- * of 128, 9 x 2048, K 17408 81 / 104 / 36, K 8192 44 / 48 / 19, K 5120 32 / 30 / -; groups of 64,
- * 9 x 5120, K 17408 85 / 90 / 68; 4-bit bf16, groups of 64, 9 x 5120, K 17408 (more than one
+ * of 128, 9 x 2048, K 17408 81 / 104 / 32, K 8192 44 / 48 / 17, K 5888 35 / 33 / -, below which the
+ * product is ahead of the GEMV everywhere; groups of 64, 9 x 5120, K 17408 85 / 90 / 68; 4-bit bf16, groups of 64, 9 x 5120, K 17408 (more than one
  * workgroup a CU) 72 / 61 / 63; past the GEMV's K, 4 x 40, K 24576 62 (one wave an output) / 67 /
  * 44. */
 static bool f32_long_k(int M, int N, int K, int bits, int gs, int num_cus) {
     const int64_t wgs = (int64_t)((N + 15) / 16) * ((M + 15) / 16);
-    return K >= 8192 && M <= 32 &&
+    return K >= 6144 && M <= 32 &&
            wgs <= (M <= 16 && (bits == 8 || gs == 32) ? 2 : 1) * (int64_t)num_cus;
 }
 

@@ -173,7 +173,7 @@ dfq_status dfq_interleave_gate_up(dfq_ctx* ctx, const void* gate, const void* up
  * share bf16 or fp16, bits are 4 or 8 and the group 32, 64 or 128, up to 8 rows run as that
  * GEMV where 4 rows of x fit in LDS, one launch per 4 rows (each weight row read once a launch),
  * and more rows as one matrix product on the matrix cores (its sums in another order); up to 32
- * rows of few columns over a K from 8192 that the GEMV does not take run as the calls below.
+ * rows of few columns over a K from 6144 that the GEMV does not take run as the calls below.
  * Every other call has fp32 weights, products and sums: on the fp32 matrix instruction where K and
  * the group are multiples of 32 and x and w are 16-byte aligned, else (and for few outputs at some
  * K below 2048) one wave per output element, re-reading W for every row.  M is at most 65535.
